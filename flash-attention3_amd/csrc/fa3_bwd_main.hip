@@ -2,12 +2,14 @@
 // side (job map, split plan, workspace plan, launch).  The kernels and their
 // device helpers are in fa3_bwd_main_kernel.h.
 #include "fa3_bwd_main_kernel.h"
+#include "fa3_bwd_reg_kernel.h"
 #include "fa3_job_map.h"
 #include "fa3_split_plan.h"
 
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <cmath>
 #include <memory>
 #include <mutex>
 #include <random>
@@ -276,6 +278,101 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
     return w;
 }
 
+// Which launches run the register-operand kernel, and how it cuts its jobs.
+// Work in units of 128 keys x 64 query rows of a dKV job (a dQ unit ~0.75):
+// share = a CU's part of it, longest = the longest dKV job of 128 keys
+// (group / chunks heads' query rows).  x = longest / share is what decides,
+// because two or three workgroups share a CU and each then runs at a part of
+// its speed, while bwd_main_kernel's one workgroup has the CU to itself.
+// Measured against bwd_main_kernel over 110 random shapes (bf16, both head
+// dims, causal and full, G 1..8):
+//   x <= 0.75: whole jobs (11) -6 to -40 %, halves 3 to 10 % behind them;
+//   0.75 < x <= 1.3: dKV jobs halved (21) -3 to -21 % with G > 1, where whole
+//     jobs lose up to +31 %; with G = 1 a dQ job is as long as a dKV job:
+//     both halved (22), -4 to -33 % at D 64, within 5 % at D 128, which
+//     stays with bwd_main_kernel there;
+//   x > 1.3: bwd_main_kernel, +8 to +100 % faster the fewer the jobs.
+// Full attention's jobs of a role are all alike: whole jobs that fill less
+// than two thirds of their last round of two workgroups per CU also halve
+// (B2 H12 S1792 D128: 672 jobs, -6 % whole, -11 % halved).
+RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
+#ifdef FA3_TIMELINE
+    return RegPlan{};  // the stamps are bwd_main_kernel's
+#endif
+    if (w.bal_m > 0) return RegPlan{};
+    const int group = p.heads_q / p.heads_kv, chunks = std::max(w.hs_chunks, 1);
+    const double qt = p.seqlen / 64;  // even: the sequence is whole 128-row tiles
+    const double units = p.causal ? 0.25 * qt * (qt + 2.0) : 0.5 * qt * qt;
+    const double share = (double)p.batch * p.heads_q * units * 1.75 / kHeadSplitCus;
+    const double x = (double)(group / chunks) * qt / share;
+    if (x > 1.3) return RegPlan{};
+    if (x > (p.head_dim == 64 ? 0.9 : 0.75)) {
+        if (group > 1) return RegPlan{2, 1};
+        return p.head_dim == 64 ? RegPlan{2, 2} : RegPlan{};
+    }
+    if (!p.causal && p.head_dim == 128) {
+        const double rounds =
+            (double)p.batch * p.heads_kv * (chunks + group) * (p.seqlen / 128) / (2 * kHeadSplitCus);
+        if (rounds > 1.0 && std::ceil(rounds) / rounds > 1.5) return RegPlan{2, 1};
+    }
+    return RegPlan{1, 1};
+}
+
+// The register-operand kernel's arguments, from a default-plan launch's.
+RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim) {
+    RegArgs r{};
+    r.q = a.q;
+    r.k = a.k;
+    r.v = a.v;
+    r.dout = a.dout;
+    r.nlse2 = a.nlse2;
+    r.ndelta = a.ndelta;
+    r.dq = a.dq;
+    r.dq_f32 = a.out_f32;
+    r.q_rs = a.q_rs;
+    r.q_hs = a.q_hs;
+    r.kv_rs = a.kv_rs;
+    r.kv_hs = a.kv_hs;
+    r.seqlen = a.seqlen;
+    r.heads_q = a.heads_q;
+    r.heads_kv = a.heads_kv;
+    r.group = a.group;
+    if (a.part_dk != nullptr) {  // head split: fp32 contributions [B][Hkv chunks][S][D]
+        r.chunks = a.hs_chunks;
+        r.heads = a.hs_heads;
+        r.dk = a.part_dk;
+        r.dv = a.part_dv;
+        r.dkv_f32 = 1;
+        r.o_rs = head_dim;
+        r.o_hs = a.seqlen * head_dim;
+        r.o_heads = a.heads_kv * a.hs_chunks;
+    } else {
+        r.chunks = 1;
+        r.heads = a.group;
+        r.dk = a.dk;
+        r.dv = a.dv;
+        r.dkv_f32 = a.out_f32;
+        r.o_rs = a.kv_rs;
+        r.o_hs = a.kv_hs;
+        r.o_heads = a.heads_kv;
+    }
+    r.scale_log2 = a.scale_log2;
+    r.scale = a.scale;
+    r.n_groups = a.n_groups;
+    r.jobs_per_group =
+        a.seqlen / 128 * (plan.split_kv * r.chunks + plan.split_q * r.group);
+    // Always position by position across an XCD's groups, longest jobs first:
+    // the hardware deals the jobs out in this order, and with small
+    // workgroups a late long job costs more than the L2 gains from one group
+    // at a time (P4 1 029 -> 866 us, B4 H16 S1024 95.9 -> 71.4, B4 H16 S2048
+    // 267.8 -> 240.7, B1 H16 S8192 783 -> 771).
+    set_job_map_with(r, [](int) { return true; });
+    r.div_hkv = a.div_hkv;
+    r.div_group = a.div_group;
+    r.div_chunks = make_fastdiv(r.chunks);
+    return r;
+}
+
 hipError_t launch_component(const BwdProblem& p, const BwdTensors& t, int role) {
     FusedArgs a = base_args(p, t);
     a.packed = t.packed_in;
@@ -394,7 +491,14 @@ hipError_t launch_backward(const BwdProblem& p, const BwdTensors& t, void* works
             a.split_desc[id] = split_desc(kind, x, g, len, sfield);
         }
     }
-    if (g_debug_kernels.load()) launch_race_check(a, p.head_dim, p.causal, p.bf16, t.stream);
+    const RegPlan reg = reg_plan(p, plan);
+    if (reg.split_kv > 0) {
+        const RegArgs r = reg_args(a, reg, p.head_dim);
+        if (g_debug_kernels.load())
+            launch_reg_race_check(r, reg, p.head_dim, p.causal, p.bf16, t.stream);
+        else launch_reg_kernel<false>(r, reg, p.head_dim, p.causal, p.bf16, t.stream);
+    }
+    else if (g_debug_kernels.load()) launch_race_check(a, p.head_dim, p.causal, p.bf16, t.stream);
     else if (p.head_dim == 128) launch_dd<128, false>(a, p.causal, p.bf16, t.stream);
     else launch_dd<64, false>(a, p.causal, p.bf16, t.stream);
     err = hipGetLastError();

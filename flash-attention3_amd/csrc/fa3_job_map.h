@@ -26,24 +26,21 @@ inline constexpr int kInterleaveJobsPerCu = 8;
 inline constexpr double kInterleaveTail = 2.0;
 inline constexpr int kInterleaveSpan = 4;
 
-// XCD-aware job map: n_groups groups of jobs_per_group jobs.  longest:
-// the longest job, share: a CU's share of the work (both in dKV steps),
-// cus: the CU count -- for the interleave choice above (the defaults: one
-// group after another).
-inline void set_job_map(FusedArgs& a, double longest = 0.0, double share = 1.0, int cus = 0) {
+// XCD-aware job map of a.n_groups groups of a.jobs_per_group jobs, an XCD's
+// groups one after another or interleaved (A: FusedArgs, or RegArgs of
+// fa3_bwd_reg_kernel.h).
+template <typename A, typename Choose>
+inline void set_job_map_with(A& a, Choose&& interleave_of) {
     int gcd8 = 8;
     while (a.n_groups % gcd8 != 0) gcd8 >>= 1;
     const int parts = 8 / gcd8;  // smallest split with n_groups * parts % 8 == 0
     const bool fits = a.jobs_per_group % parts == 0;
     a.xcd_parts = fits ? parts : 0;
     a.xcd_vgroups = fits ? a.n_groups * parts / 8 : 0;
-    const long long jobs = (long long)a.n_groups * a.jobs_per_group;
     // the groups an XCD's virtual groups belong to (one more where its
     // first part is not a group's first)
     const int span = fits ? (a.xcd_vgroups + parts - 1) / parts : a.n_groups;
-    const bool interleave =
-        jobs <= (long long)kInterleaveJobsPerCu * cus ||
-        (span <= kInterleaveSpan && longest * a.xcd_vgroups >= kInterleaveTail * share);
+    const bool interleave = interleave_of(span);
     a.xcd_interleave = interleave ? 1 : 0;
     a.xcd_mode = a.xcd_parts | a.xcd_interleave << 8;
     a.map_radix = !fits ? 0 : interleave ? a.xcd_vgroups : a.jobs_per_group / parts;
@@ -51,6 +48,17 @@ inline void set_job_map(FusedArgs& a, double longest = 0.0, double share = 1.0, 
     a.div_radix = make_fastdiv(a.map_radix);
     a.div_jpg = make_fastdiv(a.jobs_per_group);
     a.div_groups = make_fastdiv(a.n_groups);
+}
+
+// The map of bwd_main_kernel's plans.  longest: the longest job, share: a
+// CU's share of the work (both in dKV steps), cus: the CU count -- for the
+// interleave choice above (the defaults: one group after another).
+inline void set_job_map(FusedArgs& a, double longest = 0.0, double share = 1.0, int cus = 0) {
+    set_job_map_with(a, [&](int span) {
+        const long long jobs = (long long)a.n_groups * a.jobs_per_group;
+        return jobs <= (long long)kInterleaveJobsPerCu * cus ||
+               (span <= kInterleaveSpan && longest * a.xcd_vgroups >= kInterleaveTail * share);
+    });
 }
 
 }  // namespace fa3

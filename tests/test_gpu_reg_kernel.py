@@ -1,0 +1,56 @@
+"""The register-operand main kernel (bwd_reg_kernel) at the edges of the
+shapes that reach it: a single 128-row tile, odd tile counts, group counts
+without XCD-aligned parts, each way of cutting the jobs (whole, dKV halved,
+both halved), fp32 head-split contributions, bf16, BSHD and a scale above
+ln 2.  Each case against the CPU oracle under the bar of gpu_util.check,
+bitwise repeatable, and bit for bit equal to its race-check instantiation
+(every job on an LDS of NaN bytes, a full wait and a barrier around every
+phase)."""
+import numpy as np
+import pytest
+
+import fa3_oracle as O
+import shaobo_fa3 as F
+from gpu_util import check, log, run_v2
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, Hq, Hkv, S, D, causal, dtype, bshd, scale; longest dKV job / a CU's share
+    (8, 25, 25, 128, 128, True, "fp16", False, None),   # one tile, whole jobs (0.73)
+    (4, 33, 33, 256, 128, True, "bf16", True, None),    # whole jobs, BSHD (0.74)
+    (2, 49, 49, 384, 128, True, "fp16", False, 1.0),    # odd tiles and groups, unscaled range (0.75)
+    (2, 33, 33, 384, 64, False, "bf16", False, None),   # D 64, full (0.74)
+    (4, 64, 32, 128, 128, True, "bf16", False, None),   # dKV jobs halved, one tile (1.14)
+    (4, 16, 8, 1024, 128, True, "fp16", True, None),    # dKV jobs halved, BSHD (1.02)
+    (4, 48, 12, 384, 64, False, "fp16", False, None),   # dKV jobs halved, D 64, full (1.02)
+    (4, 20, 5, 384, 128, True, "bf16", False, None),    # head split in 4 chunks, halved (0.91)
+    (3, 16, 2, 384, 64, False, "fp16", True, None),     # head split in 8 chunks, D 64 (1.02)
+    (2, 12, 12, 1792, 128, False, "bf16", False, None), # full, last round nearly empty: halved
+    (3, 21, 21, 384, 64, True, "fp16", False, None),    # both roles halved, D 64 (1.16)
+    (3, 19, 19, 128, 64, True, "bf16", False, 1.0),     # few jobs: bwd_main_kernel (2.57)
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,dtype,bshd,scale", CASES)
+def test_reg_kernel(B, Hq, Hkv, S, D, causal, dtype, bshd, scale):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    log(f"[case] reg kernel B={B} Hq={Hq} Hkv={Hkv} S={S} D={D} causal={causal} {dtype} "
+        f"bshd={bshd} scale={scale}")
+    lib = F.load()
+    kw = {} if scale is None else {"scale": scale}
+    g = O.golden(B, Hq, Hkv, S, D, causal, dtype=dtype, **kw)
+    res = run_v2(g, torch, bshd=bshd)
+    assert res["status"] == F.SUCCESS, F.status_name(res["status"])
+    check(res, g)
+    again = run_v2(g, torch, bshd=bshd)
+    lib.shaobo_fa3_ext_set_race_check(1)
+    try:
+        slow = run_v2(g, torch, bshd=bshd)
+    finally:
+        lib.shaobo_fa3_ext_set_race_check(0)
+    for n in ("dq", "dk", "dv", "delta"):
+        np.testing.assert_array_equal(again[n], res[n], err_msg=n)
+        np.testing.assert_array_equal(slow[n], res[n], err_msg=n)
