@@ -281,41 +281,62 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 // Which launches run the register-operand kernel, and how it cuts its jobs.
 // Work in units of 128 keys x 64 query rows of a dKV job (a dQ unit ~0.75):
 // share = a CU's part of it, longest = the longest dKV job of 128 keys
-// (group / chunks heads' query rows).  x = longest / share is what decides,
-// because two or three workgroups share a CU and each then runs at a part of
-// its speed, while bwd_main_kernel's one workgroup has the CU to itself.
-// Measured against bwd_main_kernel over 110 random shapes (bf16, both head
-// dims, causal and full, G 1..8):
-//   x <= 0.75: whole jobs (11) -6 to -40 %, halves 3 to 10 % behind them;
-//   0.75 < x <= 1.3: dKV jobs halved (21) -3 to -21 % with G > 1, where whole
-//     jobs lose up to +31 %; with G = 1 a dQ job is as long as a dKV job:
-//     both halved (22), -4 to -33 % at D 64, within 5 % at D 128, which
-//     stays with bwd_main_kernel there;
-//   x > 1.3: bwd_main_kernel, +8 to +100 % faster the fewer the jobs.
-// Full attention's jobs of a role are all alike: whole jobs that fill less
-// than two thirds of their last round of two workgroups per CU also halve
-// (B2 H12 S1792 D128: 672 jobs, -6 % whole, -11 % halved).
+// (group / chunks heads' query rows).  x = longest / share decides between
+// the kernels, because two (D 128) or three (D 64) workgroups share a CU and
+// each then runs at a part of its speed, while bwd_main_kernel's one
+// workgroup has the CU to itself.  Measured against bwd_main_kernel over 110
+// random shapes (bf16, both head dims, causal and full, G 1..8):
+//   x <= 0.75: -6 to -40 %;
+//   0.75 < x <= 1.3: G > 1 -3 to -21 % (with its longest dKV jobs halved,
+//     below); with G = 1 a dQ job is as long as a dKV job: both halved, -4 to
+//     -33 % at D 64, within 5 % at D 128, which stays with bwd_main_kernel;
+//   x > 1.3: bwd_main_kernel, 8 to 100 % faster the fewer the jobs.
+// A dKV job longer than a workgroup slot's share sets the launch's end: such
+// tiles run as two jobs of 64 keys, at ~10 % more per unit.  Causal, only the
+// longest tiles (B2 Hq32 Hkv8 S2048 D128, of 16 tiles 0 / 4 / 8 / 12 / 16
+// halved: 315 / 263 / 233 / 236 / 245 us, the rule 9; B1 Hq32 Hkv1 S4096, of
+// 32 tiles 0 / 8 / 16 / 20 / 32: 622 / 510 / 449 / 431 / 451, the rule 18; B2
+// Hq32 Hkv8 S4096 within 1 % from 0 to 12, the rule 4).  Against whole or all
+// halved by x alone, with the longest jobs at raised priority: B4 Hq20 Hkv5
+// S384 40.4 -> 36.5 us, B1 Hq32 Hkv16 S3328 296.2 -> 287.5, B2 Hq32 Hkv8 S2048
+// 221.9 -> 219.8, S4096 827.9 -> 820.2, B4 Hq12 Hkv3 S2304 229.1 -> 230.5; the
+// priority alone is worth at most 1.5 % either way and went.
+// Full attention's jobs of a role are all alike, so all are halved or none;
+// whole jobs that fill less than two thirds of their last round of two
+// workgroups per CU also halve (B2 H12 S1792 D128: 672 jobs, -6 % whole, -11 %
+// halved).
 RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
+    RegPlan r;
 #ifdef FA3_TIMELINE
-    return RegPlan{};  // the stamps are bwd_main_kernel's
+    return r;  // the stamps are bwd_main_kernel's
 #endif
-    if (w.bal_m > 0) return RegPlan{};
+    if (w.bal_m > 0) return r;
     const int group = p.heads_q / p.heads_kv, chunks = std::max(w.hs_chunks, 1);
-    const double qt = p.seqlen / 64;  // even: the sequence is whole 128-row tiles
+    const int heads = group / chunks, qt = p.seqlen / 64;  // (qt even)
     const double units = p.causal ? 0.25 * qt * (qt + 2.0) : 0.5 * qt * qt;
     const double share = (double)p.batch * p.heads_q * units * 1.75 / kHeadSplitCus;
-    const double x = (double)(group / chunks) * qt / share;
-    if (x > 1.3) return RegPlan{};
-    if (x > (p.head_dim == 64 ? 0.9 : 0.75)) {
-        if (group > 1) return RegPlan{2, 1};
-        return p.head_dim == 64 ? RegPlan{2, 2} : RegPlan{};
+    const double x = (double)heads * qt / share;
+    if (x > 1.3) return r;
+    if (group == 1 && x > (p.head_dim == 64 ? 0.9 : 0.75)) {
+        r.on = p.head_dim == 64;
+        r.split_kv = r.split_q = 2;
+        return r;
     }
-    if (!p.causal && p.head_dim == 128) {
-        const double rounds =
-            (double)p.batch * p.heads_kv * (chunks + group) * (p.seqlen / 128) / (2 * kHeadSplitCus);
-        if (rounds > 1.0 && std::ceil(rounds) / rounds > 1.5) return RegPlan{2, 1};
+    r.on = true;
+    const double slot = share / (p.head_dim == 64 ? 3 : 2);
+    if (p.causal) {
+        // tile k's job: heads x (qt - 2 k) units
+        const double k = 0.5 * (qt - slot / heads);
+        r.split_kv = 0;
+        r.halved = std::min(std::max((int)std::ceil(k), 0), qt / 2);
+    } else {
+        const double rounds = (double)p.batch * p.heads_kv * (chunks + group) * (qt / 2) /
+                              (2 * kHeadSplitCus);
+        if (x > 0.9 ||
+            (p.head_dim == 128 && rounds > 1.0 && std::ceil(rounds) / rounds > 1.5))
+            r.split_kv = 2;
     }
-    return RegPlan{1, 1};
+    return r;
 }
 
 // The register-operand kernel's arguments, from a default-plan launch's.
@@ -360,7 +381,9 @@ RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim) {
     r.scale = a.scale;
     r.n_groups = a.n_groups;
     r.jobs_per_group =
-        a.seqlen / 128 * (plan.split_kv * r.chunks + plan.split_q * r.group);
+        a.seqlen / 128 * (std::max(plan.split_kv, 1) * r.chunks + plan.split_q * r.group) +
+        plan.halved * r.chunks;
+    r.halved = plan.halved;
     // Always position by position across an XCD's groups, longest jobs first:
     // the hardware deals the jobs out in this order, and with small
     // workgroups a late long job costs more than the L2 gains from one group
@@ -492,7 +515,7 @@ hipError_t launch_backward(const BwdProblem& p, const BwdTensors& t, void* works
         }
     }
     const RegPlan reg = reg_plan(p, plan);
-    if (reg.split_kv > 0) {
+    if (reg.on) {
         const RegArgs r = reg_args(a, reg, p.head_dim);
         if (g_debug_kernels.load())
             launch_reg_race_check(r, reg, p.head_dim, p.causal, p.bf16, t.stream);

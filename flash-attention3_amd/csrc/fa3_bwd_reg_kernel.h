@@ -44,10 +44,13 @@
 namespace fa3 {
 
 // How a launch cuts its jobs: keys of a dKV job = 128 / split_kv, query rows
-// of a dQ job = 128 / split_q.  split_kv 0: the launch runs bwd_main_kernel.
+// of a dQ job = 128 / split_q.  split_kv 0 (causal): the first `halved` of the
+// 128-key tiles, the longest, as two 64-key jobs, the others whole.
 struct RegPlan {
-    int split_kv = 0;
-    int split_q = 0;
+    bool on = false;  // false: the launch runs bwd_main_kernel
+    int split_kv = 1;
+    int split_q = 1;
+    int halved = 0;
 };
 
 struct RegArgs {
@@ -66,6 +69,7 @@ struct RegArgs {
     int seqlen, heads_q, heads_kv, group;
     int heads;   // query heads a dKV job streams: group / chunks
     int chunks;  // dKV jobs per key tile
+    int halved;  // kSplitKv 0: the first `halved` 128-key tiles run as 64-key jobs
     float scale_log2, scale;
     // job map (job_of)
     int n_groups, jobs_per_group, map_radix, xcd_parts, xcd_interleave, xcd_vgroups, xcd_mode;
@@ -307,8 +311,8 @@ __device__ __forceinline__ void reg_add(const FA3_LDS char* slot, f32x4 (*acc)[2
 
 // Key tile kt (128 / kSplit keys) of KV head hkv in batch b, streaming the
 // query tiles of `heads` query heads from h0 on; out head ho.
-template <int D, bool kCausal, bool kBf16, int kSplit, bool kDebug>
-__device__ __forceinline__ void reg_dkv(const RegArgs& a, int b, int hkv, int kt, int h0, int ho,
+template <int D, bool kCausal, bool kBf16, int kSplit, bool kDebug, typename A>
+__device__ __forceinline__ void reg_dkv(const A& a, int b, int hkv, int kt, int h0, int ho,
                                         FA3_LDS char* smem) {
     using C = RegCfg<D>;
     constexpr int kKb = kRegWaves / kSplit;  // 32-key blocks of the job
@@ -465,8 +469,8 @@ __device__ __forceinline__ void reg_dkv(const RegArgs& a, int b, int hkv, int kt
 }
 
 // Query tile qt (128 / kSplit rows) of query head hq (KV head hkv) in batch b.
-template <int D, bool kCausal, bool kBf16, int kSplit, bool kDebug>
-__device__ __forceinline__ void reg_dq(const RegArgs& a, int b, int hq, int hkv, int qt,
+template <int D, bool kCausal, bool kBf16, int kSplit, bool kDebug, typename A>
+__device__ __forceinline__ void reg_dq(const A& a, int b, int hq, int hkv, int qt,
                                        FA3_LDS char* smem) {
     using C = RegCfg<D>;
     constexpr int kQb = kRegWaves / kSplit;  // 32-row blocks of the job
@@ -617,7 +621,10 @@ __global__ __launch_bounds__(kRegThreads, D == 64 ? 3 : 2) void bwd_reg_kernel(R
     int g, pos;
     job_of(a, id, g, pos);
     const int b = fdiv(a.div_hkv, g), hkv = g - b * a.heads_kv;
-    const int QTk = a.seqlen / (128 / kSplitKv), QTq = a.seqlen / (128 / kSplitQ);
+    const int QT = a.seqlen / 128, QTq = a.seqlen / (128 / kSplitQ);
+    // 64-key tiles in front, 128-key tiles behind them
+    const int n64 = kSplitKv == 2 ? 2 * QT : kSplitKv == 0 ? 2 * a.halved : 0;
+    const int QTk = kSplitKv == 0 ? QT + a.halved : n64 > 0 ? n64 : QT;
     // the dKV jobs first, by key tile (causal: longest first), one per chunk
     // of query heads; then the dQ jobs, latest query tile first
     int level, slot;  // slot < chunks: dKV, else the dQ job of query head slot - chunks
@@ -630,22 +637,21 @@ __global__ __launch_bounds__(kRegThreads, D == 64 ? 3 : 2) void bwd_reg_kernel(R
         level = fdiv(a.div_group, r);
         slot = a.chunks + r - level * a.group;
     }
-    if constexpr (kCausal && D == 128) {
-        // The longest dKV jobs run at raised priority beside their CU's other
-        // workgroup: they set the launch's end where one is longer than a
-        // slot's share (B2 Hq32 Hkv8 S2048: 230.4 -> 223.0 us; neutral where not).
-        if (slot < a.chunks) {
-            const int x = level * 8 / QTk;
-            if (x < 1) __builtin_amdgcn_s_setprio(3);
-            else if (x < 2) __builtin_amdgcn_s_setprio(2);
-            else if (x < 4) __builtin_amdgcn_s_setprio(1);
+    const int h0 = hkv * a.group + slot * a.heads, ho = hkv * a.chunks + slot;
+    if (slot < a.chunks) {
+        if constexpr (kSplitKv == 0) {
+            // (the arguments re-read from the argument segment: held across
+            // the roles' code, they spill scalar registers)
+            typedef __attribute__((address_space(4))) const RegArgs KReg;
+            KReg* ap = (KReg*)__builtin_amdgcn_kernarg_segment_ptr();
+            __asm__ volatile("" : "+s"(ap));
+            if (level < n64) reg_dkv<D, kCausal, kBf16, 2, kDebug>(*ap, b, hkv, level, h0, ho, smem);
+            else
+                reg_dkv<D, kCausal, kBf16, 1, kDebug>(*ap, b, hkv, level - n64 / 2, h0, ho, smem);
+        } else {
+            reg_dkv<D, kCausal, kBf16, kSplitKv, kDebug>(a, b, hkv, level, h0, ho, smem);
         }
-    }
-    if (slot < a.chunks)
-        reg_dkv<D, kCausal, kBf16, kSplitKv, kDebug>(a, b, hkv, level,
-                                                     hkv * a.group + slot * a.heads,
-                                                     hkv * a.chunks + slot, smem);
-    else
+    } else
         reg_dq<D, kCausal, kBf16, kSplitQ, kDebug>(a, b, hkv * a.group + slot - a.chunks, hkv,
                                                    QTq - 1 - level, smem);
 }
@@ -660,9 +666,12 @@ void launch_reg_kernel(const RegArgs& a, RegPlan plan, int head_dim, bool causal
     auto pick = [&](auto d, auto cz, auto bf) {
         constexpr int kD = decltype(d)::value;
         constexpr bool kC = decltype(cz)::value, kB = decltype(bf)::value;
-        if (plan.split_kv == 1) go(bwd_reg_kernel<kD, kC, kB, 1, 1, kDebug>);
-        else if (plan.split_q == 1) go(bwd_reg_kernel<kD, kC, kB, 2, 1, kDebug>);
-        else go(bwd_reg_kernel<kD, kC, kB, 2, 2, kDebug>);
+        if constexpr (kD == 64) {
+            if (plan.split_q == 2) return go(bwd_reg_kernel<kD, kC, kB, 2, 2, kDebug>);
+        }
+        if constexpr (kC) go(bwd_reg_kernel<kD, kC, kB, 0, 1, kDebug>);
+        else if (plan.split_kv == 1) go(bwd_reg_kernel<kD, kC, kB, 1, 1, kDebug>);
+        else go(bwd_reg_kernel<kD, kC, kB, 2, 1, kDebug>);
     };
     auto types = [&](auto d) {
         using T = std::true_type;
