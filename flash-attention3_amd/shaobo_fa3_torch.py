@@ -8,6 +8,7 @@ stream through the library's stream entry point
 (shaobo_fa3_bwd_v2_on_stream, include/shaobo_fa3_ext.h), so it orders
 correctly with the surrounding torch work and with CUDA-graph capture of
 that stream.  A fake (meta) implementation gives shapes for tracing.
+Below its argument checks the op's body is native (csrc/fa3_torch_op.cpp).
 
 The op launches without synchronising, so a split wait that gave up (the
 library's bounded wait between two workgroups sharing one output tile) cannot
@@ -20,7 +21,10 @@ an integration example and a test vehicle; the library provides the
 backward only.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import math
+import os
 from typing import Optional, Tuple
 
 import torch
@@ -41,24 +45,46 @@ def _lib():
     return lib
 
 
+_NATIVE_PATH = os.path.join(os.path.dirname(F.LIB_PATH), "_fa3_torch.so")
+_NATIVE = None
+
+
+def _native():
+    """The native body (csrc/fa3_torch_op.cpp), or False where it has not been
+    built (`make -C flash-attention3_amd torch`): then the same body runs in
+    Python through ctypes."""
+    global _NATIVE
+    if _NATIVE is None:
+        if os.path.exists(_NATIVE_PATH):
+            loader = importlib.machinery.ExtensionFileLoader("_fa3_torch", _NATIVE_PATH)
+            spec = importlib.util.spec_from_loader("_fa3_torch", loader)
+            mod = importlib.util.module_from_spec(spec)
+            loader.exec_module(mod)
+            _NATIVE = mod.backward
+        else:
+            _NATIVE = False
+    return _NATIVE
+
+
 def _check(dout, q, k, v, out, lse):
-    if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape or out.shape != q.shape \
-            or dout.shape != q.shape:
+    qs, ks = q.shape, k.shape
+    if len(qs) != 4 or len(ks) != 4 or v.shape != ks or out.shape != qs or dout.shape != qs:
         raise ValueError("expected BHSD tensors: q, out, dout [B, Hq, S, D], k, v [B, Hkv, S, D]")
-    B, Hq, S, D = q.shape
-    if k.shape[0] != B or k.shape[2] != S or k.shape[3] != D or Hq % k.shape[1]:
+    B, Hq, S, D = qs
+    if ks[0] != B or ks[2] != S or ks[3] != D or Hq % ks[1]:
         raise ValueError("k / v shape does not match q")
     if lse.shape != (B, Hq, S) or lse.dtype != torch.float32:
         raise ValueError("softmax_lse must be fp32 [B, Hq, S]")
-    if q.dtype not in (torch.float16, torch.bfloat16):
+    dt = q.dtype
+    if dt not in (torch.float16, torch.bfloat16):
         raise ValueError("q, k, v, out, dout must be fp16 or bf16")
-    for t in (dout, k, v, out):
-        if t.dtype != q.dtype:
-            raise ValueError("q, k, v, out, dout must share one dtype")
+    if dout.dtype != dt or k.dtype != dt or v.dtype != dt or out.dtype != dt:
+        raise ValueError("q, k, v, out, dout must share one dtype")
+    dev = q.device
     for t in (dout, q, k, v, out, lse):
         if not t.is_contiguous():
             raise ValueError("tensors must be contiguous (BHSD)")
-        if t.device != q.device or t.device.type != "cuda":
+        if t.device != dev or dev.type != "cuda":
             raise ValueError("tensors must be on the same GPU")
 
 
@@ -71,6 +97,15 @@ def flash_attn_backward(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v:
     """(dQ, dK, dV, softmax_d) of softmax(scale Q K^T) V given dO, O and the
     natural-log LSE; fp16 or bf16 BHSD in and out, softmax_d fp32 [B, Hq, S]."""
     _check(dout, q, k, v, out, softmax_lse)
+    native = _native()
+    if native:
+        idx = q.device.index
+        if idx == torch.cuda.current_device():
+            return native(dout, q, k, v, out, softmax_lse, causal, softmax_scale, deterministic,
+                          torch._C._cuda_getCurrentRawStream(idx))
+        with torch.cuda.device(idx):
+            return native(dout, q, k, v, out, softmax_lse, causal, softmax_scale, deterministic,
+                          torch._C._cuda_getCurrentRawStream(idx))
     lib = _lib()
     B, Hq, S, D = q.shape
     p = F.make_params(lib, batch=B, seqlen=S, heads_q=Hq, heads_kv=k.shape[1], head_dim=D,
