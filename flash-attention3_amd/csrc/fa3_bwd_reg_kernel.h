@@ -360,12 +360,10 @@ __device__ __forceinline__ void reg_dkv(const A& a, int b, int hkv, int kt, int 
     const int qa = kCausal ? (kt * kKb) >> 1 : 0, qb = S / 64;
     const int n_it = a.heads * (qb - qa);
 
-    int ld_qt = qa;
-    size_t ld_e = q_elem<D>(a, b, h0, qa * 64);
-    size_t ld_row = ((size_t)b * a.heads_q + h0) * S + qa * 64;
+    int ld_h = 0;
+    size_t ld_e = q_elem<D>(a, b, h0, (qb - 1) * 64);
+    size_t ld_row = ((size_t)b * a.heads_q + h0) * S + (qb - 1) * 64;
     const size_t step_e = (size_t)64 * a.q_rs;
-    const size_t wrap_e = (size_t)a.q_hs - (size_t)(qb - qa - 1) * step_e;
-    const size_t wrap_row = (size_t)S - (size_t)(qb - qa - 1) * 64;
     auto issue = [&](FA3_LDS char* st) {
         const int ln = opaque_tid() & 63;
         const uint32_t off = reg_load_off<D>(ln, a.q_rs);
@@ -375,13 +373,12 @@ __device__ __forceinline__ void reg_dkv(const A& a, int b, int hkv, int kt, int 
             __builtin_amdgcn_global_load_lds(
                 (const void*)((w == 0 ? a.nlse2 : a.ndelta) + ld_row + ln),
                 (FA3_LDS void*)(st + 2 * C::kTileBytes + 256 * w), 4, 0, 0);
-        if (++ld_qt == qb) {
-            ld_qt = qa;
-            ld_e += wrap_e;
-            ld_row += wrap_row;
-        } else {
-            ld_e += step_e;
-            ld_row += 64;
+        ld_e += (size_t)a.q_hs;
+        ld_row += (size_t)S;
+        if (++ld_h == a.heads) {
+            ld_h = 0;
+            ld_e -= (size_t)a.heads * a.q_hs + step_e;
+            ld_row -= (size_t)a.heads * S + 64;
         }
     };
     FA3_LDS char* s0 = smem;
@@ -407,8 +404,8 @@ __device__ __forceinline__ void reg_dkv(const A& a, int b, int hkv, int kt, int 
     const int rsub = 32 * rs;  // this wave's rows of a stage: all (kSplit 1), or 32 from here
     const RegReader<D> rd0(lane, rsub);
     const float c = a.scale_log2;
-    const int r_first = qa * 64 + rsub - key0;
-    int row0 = r_first;  // this wave's first row of the stage relative to its first key
+    int row0 = (qb - 1) * 64 + rsub - key0;  // this wave's first row of the stage relative to
+    int head = 0;                            // its first key; the stage's head
 
     auto sub = [&](const FA3_LDS char* st, int r) {
         RegReader<D> rd = rd0;
@@ -467,8 +464,10 @@ __device__ __forceinline__ void reg_dkv(const A& a, int b, int hkv, int kt, int 
         sub(st, 0);
         if constexpr (kSplit == 1) sub(st, 1);
         if (kCausal) {
-            row0 += 64;
-            if (row0 + key0 >= S) row0 = r_first;  // next query head
+            if (++head == a.heads) {  // next query tile
+                head = 0;
+                row0 -= 64;
+            }
         }
     };
     for (;;) {
