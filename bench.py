@@ -119,6 +119,12 @@ class Hip:
         assert self.lib.hipDeviceSynchronize() == 0
 
 
+# The kernel behind the main stage (key "bwd_main_kernel" of the times) of
+# each configuration; another --shape runs either of the two.
+MAIN_KERNEL = {"P1": "bwd_main_kernel", "P2": "bwd_main_kernel", "P3": "bwd_main_kernel",
+               "P4": "bwd_reg_kernel", "P5": "bwd_reg_kernel"}
+
+
 def load_traffic(config):
     """HBM bytes per launch of the main kernel, measured with rocprofv3
     FETCH_SIZE / WRITE_SIZE and scaled by a copy kernel of known size
@@ -365,7 +371,7 @@ def measure(torch, lib, F, hip, name, steps, warmup, deterministic, dtype="fp16"
         "kernels_ms_marked": {"preprocess_kernel": round(pre_marked, 5),
                               "bwd_main_kernel": round(main_marked, 5),
                               "ms_per_step": round(staged_ms, 5)},
-        "roofline": {"kernel": "bwd_main_kernel", "bound": "mfma",
+        "roofline": {"kernel": MAIN_KERNEL.get(name, "main kernel"), "bound": "mfma",
                      "achieved": round(main_tflops, 3),
                      "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(main_tflops / FP16_PEAK_TFLOPS, 5),
