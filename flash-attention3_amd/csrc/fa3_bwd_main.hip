@@ -387,8 +387,10 @@ RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim) {
     // Always position by position across an XCD's groups, longest jobs first:
     // the hardware deals the jobs out in this order, and with small
     // workgroups a late long job costs more than the L2 gains from one group
-    // at a time (P4 1 029 -> 866 us, B4 H16 S1024 95.9 -> 71.4, B4 H16 S2048
-    // 267.8 -> 240.7, B1 H16 S8192 783 -> 771).
+    // at a time (B2 Hq32 Hkv8 S4096 D128 causal 1 029 -> 866 us, B4 H16 S1024
+    // 95.9 -> 71.4, B4 H16 S2048 267.8 -> 240.7, B1 H16 S8192 783 -> 771; full
+    // attention, B2 H12 S1664 D64 70.9 -> 63.8, B2 H16 S8192 D64 equal though
+    // five times the algorithmic bytes are fetched).
     set_job_map_with(r, [](int) { return true; });
     r.div_hkv = a.div_hkv;
     r.div_group = a.div_group;
