@@ -461,6 +461,19 @@ int shaobo_fa3_ext_bwd_v2_stages(const void* dout, const void* q, const void* k,
                         params, opt);
 }
 
+int shaobo_fa3_ext_bwd_v2_plan(const ShaoboFa3Params* params, ShaoboFa3ExtPlan* plan) {
+    const int status = validate(params);
+    if (status != SHAOBO_FA3_STATUS_SUCCESS) return status;
+    if (plan == nullptr || plan->struct_size < sizeof(ShaoboFa3ExtPlan)) {
+        return SHAOBO_FA3_STATUS_INVALID_VALUE;
+    }
+    const fa3::BwdProblem pr = problem_of(params);
+    const fa3::WorkspacePlan w = fa3::plan_workspace(pr);
+    if (!w.ok) return SHAOBO_FA3_STATUS_INVALID_VALUE;
+    fa3::describe_launch(pr, w, plan);
+    return SHAOBO_FA3_STATUS_SUCCESS;
+}
+
 int shaobo_fa3_ext_split_status(const void* workspace, void* stream) {
     const hipStream_t s = static_cast<hipStream_t>(stream);
     int device = -1;

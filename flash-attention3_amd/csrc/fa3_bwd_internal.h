@@ -138,6 +138,10 @@ struct WorkspacePlan {
 
 WorkspacePlan plan_workspace(const BwdProblem& p);
 
+// What launch_backward would run for p under plan w (plan_workspace(p)), for
+// shaobo_fa3_ext_bwd_v2_plan.
+void describe_launch(const BwdProblem& p, const WorkspacePlan& w, ShaoboFa3ExtPlan* out);
+
 // Launches the backward on t.stream: the delta / lse2 preprocess (or the
 // packed sidecar's fold), then the main kernel.  *epoch receives the value
 // the launch's split waits compare with (and write into the error word when

@@ -18,8 +18,6 @@
 namespace fa3 {
 namespace {
 
-
-
 FusedArgs base_args(const BwdProblem& p, const BwdTensors& t) {
     FusedArgs a{};
     a.q = (const _Float16*)t.q;
@@ -48,7 +46,6 @@ FusedArgs base_args(const BwdProblem& p, const BwdTensors& t) {
     a.spin_limit = 1;
     return a;
 }
-
 
 std::atomic<int> g_spin_limit{1 << 24};
 std::atomic<bool> g_debug_kernels{false};
@@ -380,22 +377,38 @@ RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim) {
     r.scale_log2 = a.scale_log2;
     r.scale = a.scale;
     r.n_groups = a.n_groups;
-    r.jobs_per_group =
-        a.seqlen / 128 * (std::max(plan.split_kv, 1) * r.chunks + plan.split_q * r.group) +
-        plan.halved * r.chunks;
     r.halved = plan.halved;
-    // Always position by position across an XCD's groups, longest jobs first:
-    // the hardware deals the jobs out in this order, and with small
-    // workgroups a late long job costs more than the L2 gains from one group
-    // at a time (B2 Hq32 Hkv8 S4096 D128 causal 1 029 -> 866 us, B4 H16 S1024
-    // 95.9 -> 71.4, B4 H16 S2048 267.8 -> 240.7, B1 H16 S8192 783 -> 771; full
-    // attention, B2 H12 S1664 D64 70.9 -> 63.8, B2 H16 S8192 D64 equal though
-    // five times the algorithmic bytes are fetched).
-    set_job_map_with(r, [](int) { return true; });
+    set_reg_job_map(r, plan);
     r.div_hkv = a.div_hkv;
     r.div_group = a.div_group;
     r.div_chunks = make_fastdiv(r.chunks);
     return r;
+}
+
+void describe_launch(const BwdProblem& p, const WorkspacePlan& w, ShaoboFa3ExtPlan* out) {
+    const int group = p.heads_q / p.heads_kv, chunks = std::max(w.hs_chunks, 1);
+    const RegPlan reg = reg_plan(p, w);
+    ShaoboFa3ExtPlan o{};
+    o.struct_size = out->struct_size;
+    o.kernel = reg.on ? SHAOBO_FA3_EXT_KERNEL_REG : SHAOBO_FA3_EXT_KERNEL_MAIN;
+    o.split_plan = w.bal_m > 0 ? 1 : 0;
+    o.chunks = chunks;
+    if (reg.on) {
+        RegArgs r{};
+        r.seqlen = p.seqlen;
+        r.group = group;
+        r.chunks = chunks;
+        r.n_groups = p.batch * p.heads_kv;
+        set_reg_job_map(r, reg);
+        o.jobs = r.n_groups * r.jobs_per_group;
+        o.split_kv = reg.split_kv;
+        o.halved = reg.halved;
+        o.split_q = reg.split_q;
+        o.xcd_parts = r.xcd_parts;
+    } else {
+        o.jobs = p.batch * p.heads_kv * (p.seqlen / kTileN) * (chunks + group);
+    }
+    *out = o;
 }
 
 hipError_t launch_component(const BwdProblem& p, const BwdTensors& t, int role) {

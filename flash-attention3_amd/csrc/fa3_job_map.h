@@ -1,9 +1,12 @@
-// XCD-aware job map of the main kernel's default plan and of the split
+// XCD-aware job map of the main kernels' default plans and of the split
 // plan's descriptors: which (group, position) each workgroup id runs (job_of
 // in fa3_bwd_main_kernel.h reads the fields set here).  Host code.
 #pragma once
 
+#include <algorithm>
+
 #include "fa3_bwd_main_kernel.h"
+#include "fa3_bwd_reg_kernel.h"
 
 namespace fa3 {
 
@@ -59,6 +62,21 @@ inline void set_job_map(FusedArgs& a, double longest = 0.0, double share = 1.0, 
         return jobs <= (long long)kInterleaveJobsPerCu * cus ||
                (span <= kInterleaveSpan && longest * a.xcd_vgroups >= kInterleaveTail * share);
     });
+}
+
+// The map of bwd_reg_kernel's launches (seqlen, group, chunks and n_groups
+// set).  Always position by position across an XCD's groups, longest jobs
+// first: the hardware deals the jobs out in this order, and with small
+// workgroups a late long job costs more than the L2 gains from one group at a
+// time (B2 Hq32 Hkv8 S4096 D128 causal 1 029 -> 866 us, B4 H16 S1024 95.9 ->
+// 71.4, B4 H16 S2048 267.8 -> 240.7, B1 H16 S8192 783 -> 771; full attention,
+// B2 H12 S1664 D64 70.9 -> 63.8, B2 H16 S8192 D64 equal though five times the
+// algorithmic bytes are fetched).
+inline void set_reg_job_map(RegArgs& r, const RegPlan& plan) {
+    r.jobs_per_group =
+        r.seqlen / 128 * (std::max(plan.split_kv, 1) * r.chunks + plan.split_q * r.group) +
+        plan.halved * r.chunks;
+    set_job_map_with(r, [](int) { return true; });
 }
 
 }  // namespace fa3

@@ -36,7 +36,7 @@ EXPORTS = (
     "shaobo_fa3_bwd_v2_on_stream", "shaobo_fa3_ext_set_split_spin_limit",
     "shaobo_fa3_ext_bwd_v2_no_alloc", "shaobo_fa3_ext_bwd_v2_timed",
     "shaobo_fa3_ext_bwd_v2_stages", "shaobo_fa3_ext_split_status",
-    "shaobo_fa3_ext_split_error_count",
+    "shaobo_fa3_ext_split_error_count", "shaobo_fa3_ext_bwd_v2_plan",
 )
 
 # Size of the static device scratch array behind shaobo_fa3_ext_bwd_v2_no_alloc
@@ -103,6 +103,16 @@ class Capabilities(ctypes.Structure):
     ]
 
 
+KERNEL_MAIN, KERNEL_REG = range(2)
+
+
+class Plan(ctypes.Structure):
+    """ShaoboFa3ExtPlan (include/shaobo_fa3_ext.h)."""
+    _fields_ = [("struct_size", ctypes.c_uint32)] + [
+        (n, ctypes.c_int32) for n in ("kernel", "split_plan", "chunks", "jobs", "split_kv",
+                                      "halved", "split_q", "xcd_parts")]
+
+
 def _declare(lib):
     P = ctypes.POINTER(Params)
     vp = ctypes.c_void_p
@@ -166,6 +176,8 @@ def load(path=LIB_PATH):
         lib.shaobo_fa3_ext_split_error_count.argtypes = [
             ctypes.c_void_p, ctypes.POINTER(ctypes.c_ulonglong)]
         lib.shaobo_fa3_ext_split_error_count.restype = ctypes.c_int
+        lib.shaobo_fa3_ext_bwd_v2_plan.argtypes = [ctypes.POINTER(Params), ctypes.POINTER(Plan)]
+        lib.shaobo_fa3_ext_bwd_v2_plan.restype = ctypes.c_int
         if path != LIB_PATH:
             return lib
         _LIB = lib
@@ -194,6 +206,15 @@ def make_params(lib=None, *, batch, seqlen, heads_q, heads_kv=None, head_dim=128
     p.deterministic = int(bool(deterministic))
     p.sync_after_launch = int(bool(sync))
     return p
+
+
+def plan_of(params):
+    """How shaobo_fa3_bwd_v2 would run `params` (a Plan; host only)."""
+    plan = Plan(struct_size=ctypes.sizeof(Plan))
+    st = load().shaobo_fa3_ext_bwd_v2_plan(ctypes.byref(params), ctypes.byref(plan))
+    if st != SUCCESS:
+        raise RuntimeError("shaobo_fa3_ext_bwd_v2_plan: " + status_name(st))
+    return plan
 
 
 def status_name(code):

@@ -126,6 +126,30 @@ int shaobo_fa3_ext_bwd_v2_stages(const void* dout,
                                  void* stream,
                                  int stages);
 
+/* How shaobo_fa3_bwd_v2 would run a shape (no counterpart in the reference):
+ * which main kernel, and how it cuts the work.  A function of the parameters
+ * alone; no HIP call is made. */
+#define SHAOBO_FA3_EXT_KERNEL_MAIN 0 /* bwd_main_kernel: 64-key and 64-row jobs */
+#define SHAOBO_FA3_EXT_KERNEL_REG 1  /* bwd_reg_kernel */
+typedef struct ShaoboFa3ExtPlan {
+    uint32_t struct_size; /* sizeof(ShaoboFa3ExtPlan), set by the caller */
+    int32_t kernel;       /* SHAOBO_FA3_EXT_KERNEL_* */
+    int32_t split_plan;   /* 1: bwd_main_kernel's split plan (jobs in two pieces) */
+    int32_t chunks;       /* dKV jobs per key tile and KV head; > 1: head split */
+    int32_t jobs;         /* jobs of the launch (split plan: workgroups) */
+    /* bwd_reg_kernel only (0 otherwise) */
+    int32_t split_kv;     /* dKV jobs of 128 / split_kv keys; 0: the first `halved` */
+    int32_t halved;       /*   128-key tiles as two jobs of 64, the others whole */
+    int32_t split_q;      /* dQ jobs of 128 / split_q rows */
+    int32_t xcd_parts;    /* parts a KV head's jobs are dealt to the XCDs in; 0: its jobs
+                           * are dealt position by position across all KV heads */
+} ShaoboFa3ExtPlan;
+
+/* Fills *plan.  Returns the status shaobo_fa3_bwd_v2_validate gives the
+ * parameters, or INVALID_VALUE for a null or short plan or a shape whose
+ * workspace size overflows. */
+int shaobo_fa3_ext_bwd_v2_plan(const ShaoboFa3Params* params, ShaoboFa3ExtPlan* plan);
+
 /* Size of the device scratch array behind shaobo_fa3_ext_bwd_v2_no_alloc:
  * 32 MiB per GPU, held from the library's first use on that GPU until the
  * process ends. */

@@ -22,6 +22,21 @@ def dev(t, torch, bshd=False):
     return x.view(torch.bfloat16) if a.dtype == np.uint16 else x
 
 
+def launch_plan(B, Hq, Hkv, S, D, causal):
+    """How the library runs a shape (shaobo_fa3_ext_bwd_v2_plan), as one word
+    group: "split" (bwd_main_kernel's split plan), "main c<chunks>", or of
+    bwd_reg_kernel "reg <dKV cut> q<split_q> c<chunks>", the dKV cut
+    "kv<split_kv>" or, causal, "h<halved 128-key tiles>/<tiles>"."""
+    p = F.plan_of(F.make_params(batch=B, seqlen=S, heads_q=Hq, heads_kv=Hkv, head_dim=D,
+                                causal=causal))
+    if p.split_plan:
+        return "split"
+    if p.kernel == F.KERNEL_MAIN:
+        return f"main c{p.chunks}"
+    cut = f"h{p.halved}/{S // 128}" if p.split_kv == 0 else f"kv{p.split_kv}"
+    return f"reg {cut} q{p.split_q} c{p.chunks}"
+
+
 def run_v2(g, torch, *, deterministic=False, with_softmax_d=True, lse=None, scale_is_set=True,
            workspace_pad=0, workspace=None, bshd=False):
     """Run shaobo_fa3_bwd_v2 on the oracle's inputs (their dtype; BSHD tensors

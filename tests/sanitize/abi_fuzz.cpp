@@ -84,6 +84,9 @@ int main(int argc, char** argv) {
         sink += shaobo_fa3_bwd_fused5_workspace_bytes(&p);
         sink += shaobo_fa3_bwd_dkv_workspace_bytes(&p);
         sink += shaobo_fa3_bwd_dq_workspace_bytes(&p);
+        ShaoboFa3ExtPlan plan;
+        plan.struct_size = (uint32_t)(rng() % 4 ? sizeof(plan) : rng() % sizeof(plan));
+        if (shaobo_fa3_ext_bwd_v2_plan(&p, &plan) == 0) sink += (size_t)plan.jobs;
         void* n = nullptr;
         // every tensor pointer null: each entry returns before launching
         sink += shaobo_fa3_bwd_v2(n, n, n, n, n, n, n, n, n, n, &p);

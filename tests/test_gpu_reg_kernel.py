@@ -11,35 +11,37 @@ import pytest
 
 import fa3_oracle as O
 import shaobo_fa3 as F
-from gpu_util import check, log, run_v2
+from gpu_util import check, launch_plan, log, run_v2
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # B, Hq, Hkv, S, D, causal, dtype, bshd, scale; longest dKV job / a CU's share
-    (8, 25, 25, 128, 128, True, "fp16", False, None),   # one tile, whole jobs (0.73)
-    (4, 33, 33, 256, 128, True, "bf16", True, None),    # whole jobs, BSHD (0.74)
-    (2, 49, 49, 384, 128, True, "fp16", False, 1.0),    # odd tiles and groups, unscaled range (0.75)
-    (2, 33, 33, 384, 64, False, "bf16", False, None),   # D 64, full (0.74)
-    (4, 64, 32, 128, 128, True, "bf16", False, None),   # dKV jobs halved, one tile (1.14)
-    (4, 16, 8, 1024, 128, True, "fp16", True, None),    # dKV jobs halved, BSHD (1.02)
-    (4, 48, 12, 384, 64, False, "fp16", False, None),   # dKV jobs halved, D 64, full (1.02)
-    (4, 20, 5, 384, 128, True, "bf16", False, None),    # head split in 4 chunks, halved (0.91)
-    (3, 16, 2, 384, 64, False, "fp16", True, None),     # head split in 8 chunks, D 64 (1.02)
-    (2, 12, 12, 1792, 128, False, "bf16", False, None), # full, last round nearly empty: halved
-    (3, 21, 21, 384, 64, True, "fp16", False, None),    # both roles halved, D 64 (1.16)
-    (3, 19, 19, 128, 64, True, "bf16", False, 1.0),     # few jobs: bwd_main_kernel (2.57)
+    # B, Hq, Hkv, S, D, causal, dtype, bshd, scale, the plan (gpu_util.launch_plan);
+    # longest dKV job / a CU's share
+    (8, 25, 25, 128, 128, True, "fp16", False, None, "reg h1/1 q1 c1"),    # one tile (0.73)
+    (4, 33, 33, 256, 128, True, "bf16", True, None, "reg h1/2 q1 c1"),     # BSHD (0.74)
+    (2, 49, 49, 384, 128, True, "fp16", False, 1.0, "reg h1/3 q1 c1"),     # odd tiles and groups, unscaled range (0.75)
+    (2, 33, 33, 384, 64, False, "bf16", False, None, "reg kv1 q1 c1"),     # D 64, full (0.74)
+    (4, 64, 32, 128, 128, True, "bf16", False, None, "reg h1/1 q1 c1"),    # one tile, G 2 (1.14)
+    (4, 16, 8, 1024, 128, True, "fp16", True, None, "reg h5/8 q1 c1"),     # BSHD (1.02)
+    (4, 48, 12, 384, 64, False, "fp16", False, None, "reg kv2 q1 c1"),     # D 64, full (1.02)
+    (4, 20, 5, 384, 128, True, "bf16", False, None, "reg h2/3 q1 c4"),     # head split (0.91)
+    (3, 16, 2, 384, 64, False, "fp16", True, None, "reg kv2 q1 c8"),       # head split, D 64 (1.02)
+    (2, 12, 12, 1792, 128, False, "bf16", False, None, "reg kv2 q1 c1"),   # 1.3 rounds of workgroups (0.44)
+    (3, 21, 21, 384, 64, True, "fp16", False, None, "reg kv2 q2 c1"),      # both roles halved, D 64 (1.16)
+    (3, 19, 19, 128, 64, True, "bf16", False, 1.0, "main c1"),             # few jobs (2.57)
 ]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,dtype,bshd,scale", CASES)
-def test_reg_kernel(B, Hq, Hkv, S, D, causal, dtype, bshd, scale):
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,dtype,bshd,scale,plan", CASES)
+def test_reg_kernel(B, Hq, Hkv, S, D, causal, dtype, bshd, scale, plan):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     log(f"[case] reg kernel B={B} Hq={Hq} Hkv={Hkv} S={S} D={D} causal={causal} {dtype} "
-        f"bshd={bshd} scale={scale}")
+        f"bshd={bshd} scale={scale}: {plan}")
     lib = F.load()
+    assert launch_plan(B, Hq, Hkv, S, D, causal) == plan
     kw = {} if scale is None else {"scale": scale}
     g = O.golden(B, Hq, Hkv, S, D, causal, dtype=dtype, **kw)
     res = run_v2(g, torch, bshd=bshd)
