@@ -285,8 +285,17 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 // random shapes (bf16, both head dims, causal and full, G 1..8):
 //   x <= 0.75: -6 to -40 %;
 //   0.75 < x <= 1.3: G > 1 -3 to -21 % (with its longest dKV jobs halved,
-//     below); with G = 1 a dQ job is as long as a dKV job: both halved, -4 to
-//     -33 % at D 64, within 5 % at D 128, which stays with bwd_main_kernel;
+//     below), but with one head per dKV job (G = 1, or a chunk per head) a dQ
+//     job is as long as a dKV job.  G = 1: both halved from 0.9 on, -4 to
+//     -33 % at D 64, within 5 % at D 128, which stays with bwd_main_kernel.
+//     A chunk per head (x in 0.75 .. 1.3, 320 shapes, dKV halved alone -> the
+//     rule, both against bwd_main_kernel): D 64 full from 1.12 on +2 to +25 %
+//     -> -5 to -10 % with both halved, causal up to +28 % -> -12 to -20 %
+//     (below S 512 dKV halved alone is 3 to 7 % faster up to 1.12);
+//     D 128 full below 1.12 -7 to -12 %, above +2 to +15 %, and causal the
+//     longer the sequence the worse (S 256, 512: -4 to -13 %; S 1024 .. 2047:
+//     -1 to -5 % below 1.12, +2 to +6 % above; S >= 2048: +1 to +19 %; S 128:
+//     +5 % above 1.12): those run bwd_main_kernel;
 //   x > 1.3: bwd_main_kernel, 8 to 100 % faster the fewer the jobs.
 // A dKV job longer than a workgroup slot's share sets the launch's end: such
 // tiles run as two jobs of 64 keys, at ~10 % more per unit.  Causal, only the
@@ -314,10 +323,18 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
     const double share = (double)p.batch * p.heads_q * units * 1.75 / kHeadSplitCus;
     const double x = (double)heads * qt / share;
     if (x > 1.3) return r;
-    if (group == 1 && x > (p.head_dim == 64 ? 0.9 : 0.75)) {
-        r.on = p.head_dim == 64;
-        r.split_kv = r.split_q = 2;
-        return r;
+    const bool d64 = p.head_dim == 64;
+    if (heads == 1) {
+        double most;
+        if (d64) most = group == 1 || p.seqlen >= 512 ? 0.9 : 1.12;
+        else if (group == 1) most = 0.75;
+        else if (!p.causal) most = 1.12;
+        else most = p.seqlen >= 2048 ? 0.75 : p.seqlen >= 1024 || p.seqlen < 256 ? 1.12 : 1.3;
+        if (x > most) {
+            r.on = d64;
+            r.split_kv = r.split_q = 2;
+            return r;
+        }
     }
     r.on = true;
     const double slot = share / (p.head_dim == 64 ? 3 : 2);

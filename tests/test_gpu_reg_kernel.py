@@ -28,6 +28,7 @@ CASES = [
     (4, 48, 12, 384, 64, False, "fp16", False, None, "reg kv2 q1 c1"),     # D 64, full (1.02)
     (4, 20, 5, 384, 128, True, "bf16", False, None, "reg h2/3 q1 c4"),     # head split (0.91)
     (3, 16, 2, 384, 64, False, "fp16", True, None, "reg kv2 q1 c8"),       # head split, D 64 (1.02)
+    (1, 20, 5, 768, 64, False, "bf16", True, None, "reg kv2 q2 c4"),       # both halved, a chunk per head (1.22)
     (2, 12, 12, 1792, 128, False, "bf16", False, None, "reg kv2 q1 c1"),   # 1.3 rounds of workgroups (0.44)
     (3, 21, 21, 384, 64, True, "fp16", False, None, "reg kv2 q2 c1"),      # both roles halved, D 64 (1.16)
     (3, 19, 19, 128, 64, True, "bf16", False, 1.0, "main c1"),             # few jobs (2.57)

@@ -20,6 +20,31 @@ def test_plan_arguments():
     assert lib.shaobo_fa3_ext_bwd_v2_plan(ctypes.byref(p), ctypes.byref(full)) == F.UNSUPPORTED
 
 
+# The lines of the rule, each with a shape on either side of it.
+RULES = [
+    # B, Hq, Hkv, S, D, causal, plan; longest dKV job / a CU's share
+    # one head per chunk: a dQ job is as long as a dKV job, as with G = 1
+    (1, 4, 1, 3968, 128, False, "main c4"),              # D 128 (1.18)
+    (1, 20, 5, 768, 128, False, "main c4"),              # (1.22)
+    (1, 44, 11, 384, 128, False, "reg kv2 q1 c4"),       # (1.11)
+    (1, 8, 2, 3584, 128, True, "main c4"),               # causal, S >= 2048 (1.26)
+    (2, 3, 1, 7808, 128, True, "main c3"),               # (0.79)
+    (2, 9, 3, 1536, 128, True, "main c3"),               # S >= 1024 (1.25)
+    (3, 8, 1, 1280, 128, True, "reg h6/10 q1 c8"),       # (1.11)
+    (1, 18, 3, 1920, 128, True, "reg h8/15 q1 c6"),      # (1.05)
+    (2, 60, 10, 128, 128, True, "main c6"),              # S < 256 (1.22)
+    (1, 36, 12, 768, 128, True, "reg h4/6 q1 c3"),       # between (1.16)
+    (1, 20, 5, 768, 64, False, "reg kv2 q2 c4"),         # D 64 (1.22)
+    (3, 24, 3, 256, 64, False, "reg kv2 q1 c8"),         # S < 512 (1.02)
+    (1, 6, 2, 5632, 64, True, "reg kv2 q2 c3"),          # (1.08)
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,plan", RULES)
+def test_rule(B, Hq, Hkv, S, D, causal, plan):
+    assert launch_plan(B, Hq, Hkv, S, D, causal) == plan
+
+
 @pytest.mark.parametrize("row", CASES, ids=lambda r: "-".join(map(str, r[:6])))
 def test_reg_kernel_rows_run_what_they_say(row):
     assert launch_plan(*row[:6]) == row[-1]
