@@ -307,6 +307,10 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 // S384 40.4 -> 36.5 us, B1 Hq32 Hkv16 S3328 296.2 -> 287.5, B2 Hq32 Hkv8 S2048
 // 221.9 -> 219.8, S4096 827.9 -> 820.2, B4 Hq12 Hkv3 S2304 229.1 -> 230.5; the
 // priority alone is worth at most 1.5 % either way and went.
+// With one head per dKV job the dQ jobs are as long and stay whole at D 128,
+// so halving dKV only adds work: none from 0.54 to 0.75 (103 shapes against
+// bwd_main_kernel: the line above 0.93 on average and up to 1.08, none halved
+// 0.84, up to 1.05; nearer 0.5 the line halves a tile or two, as fast).
 // Full attention's jobs of a role are all alike, so all are halved or none;
 // whole jobs that fill less than two thirds of their last round of two
 // workgroups per CU also halve (B2 H12 S1792 D128: 672 jobs, -6 % whole, -11 %
@@ -342,7 +346,9 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
         // tile k's job: heads x (qt - 2 k) units
         const double k = 0.5 * (qt - slot / heads);
         r.split_kv = 0;
-        r.halved = std::min(std::max((int)std::ceil(k), 0), qt / 2);
+        r.halved = heads == 1 && !d64 && x > 0.54 && x <= 0.75
+                       ? 0
+                       : std::min(std::max((int)std::ceil(k), 0), qt / 2);
     } else {
         const double rounds = (double)p.batch * p.heads_kv * (chunks + group) * (qt / 2) /
                               (2 * kHeadSplitCus);

@@ -19,9 +19,9 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # B, Hq, Hkv, S, D, causal, dtype, bshd, scale, the plan (gpu_util.launch_plan);
     # longest dKV job / a CU's share
-    (8, 25, 25, 128, 128, True, "fp16", False, None, "reg h1/1 q1 c1"),    # one tile (0.73)
-    (4, 33, 33, 256, 128, True, "bf16", True, None, "reg h1/2 q1 c1"),     # BSHD (0.74)
-    (2, 49, 49, 384, 128, True, "fp16", False, 1.0, "reg h1/3 q1 c1"),     # odd tiles and groups, unscaled range (0.75)
+    (8, 25, 25, 128, 128, True, "fp16", False, None, "reg h0/1 q1 c1"),    # one tile (0.73)
+    (4, 33, 33, 256, 128, True, "bf16", True, None, "reg h0/2 q1 c1"),     # BSHD (0.74)
+    (2, 49, 49, 384, 128, True, "fp16", False, 1.0, "reg h0/3 q1 c1"),     # odd tiles and groups, unscaled range (0.75)
     (2, 33, 33, 384, 64, False, "bf16", False, None, "reg kv1 q1 c1"),     # D 64, full (0.74)
     (4, 64, 32, 128, 128, True, "bf16", False, None, "reg h1/1 q1 c1"),    # one tile, G 2 (1.14)
     (4, 16, 8, 1024, 128, True, "fp16", True, None, "reg h5/8 q1 c1"),     # BSHD (1.02)

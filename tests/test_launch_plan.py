@@ -37,6 +37,11 @@ RULES = [
     (1, 20, 5, 768, 64, False, "reg kv2 q2 c4"),         # D 64 (1.22)
     (3, 24, 3, 256, 64, False, "reg kv2 q1 c8"),         # S < 512 (1.02)
     (1, 6, 2, 5632, 64, True, "reg kv2 q2 c3"),          # (1.08)
+    # D 128 causal, one head per dKV job: none halved
+    (1, 27, 27, 2560, 128, True, "reg h1/20 q1 c1"),     # (0.52)
+    (10, 5, 5, 1280, 128, True, "reg h1/10 q1 c1"),      # (0.53)
+    (3, 2, 2, 8832, 128, True, "reg h0/69 q1 c1"),       # (0.70)
+    (1, 11, 11, 5376, 128, True, "reg h0/42 q1 c1"),     # (0.62)
 ]
 
 
