@@ -288,6 +288,10 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 //     below), but with one head per dKV job (G = 1, or a chunk per head) a dQ
 //     job is as long as a dKV job.  G = 1: both halved from 0.9 on, -4 to
 //     -33 % at D 64, within 5 % at D 128, which stays with bwd_main_kernel.
+//     D 64 causal: from 0.6 on for S >= 512 (109 shapes of 0.6 .. 0.9, whole ->
+//     both halved against bwd_main_kernel: S >= 2048 0.97, up to 1.11 -> 0.85,
+//     up to 0.91; S 1024 .. 2047 0.91 -> 0.79; S 512 .. 1023 0.77 -> 0.72;
+//     below S 512 equal).
 //     A chunk per head (x in 0.75 .. 1.3, 320 shapes, dKV halved alone -> the
 //     rule, both against bwd_main_kernel): D 64 full from 1.12 on +2 to +25 %
 //     -> -5 to -10 % with both halved, causal up to +28 % -> -12 to -20 %
@@ -330,7 +334,8 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
     const bool d64 = p.head_dim == 64;
     if (heads == 1) {
         double most;
-        if (d64) most = group == 1 || p.seqlen >= 512 ? 0.9 : 1.12;
+        if (d64 && p.seqlen >= 512) most = p.causal ? 0.6 : 0.9;
+        else if (d64) most = group == 1 ? 0.9 : 1.12;
         else if (group == 1) most = 0.75;
         else if (!p.causal) most = 1.12;
         else most = p.seqlen >= 2048 ? 0.75 : p.seqlen >= 1024 || p.seqlen < 256 ? 1.12 : 1.3;

@@ -42,6 +42,11 @@ RULES = [
     (10, 5, 5, 1280, 128, True, "reg h1/10 q1 c1"),      # (0.53)
     (3, 2, 2, 8832, 128, True, "reg h0/69 q1 c1"),       # (0.70)
     (1, 11, 11, 5376, 128, True, "reg h0/42 q1 c1"),     # (0.62)
+    # D 64 causal, one head per dKV job: both halved from 0.6 on, S >= 512
+    (3, 2, 2, 7424, 64, True, "reg kv2 q2 c1"),          # (0.83)
+    (1, 5, 5, 8704, 64, True, "reg kv2 q2 c1"),          # (0.85)
+    (2, 4, 4, 8064, 64, True, "reg h27/63 q1 c1"),       # (0.57)
+    (6, 23, 23, 256, 64, True, "reg h2/2 q1 c1"),        # S < 512 (0.71)
 ]
 
 
