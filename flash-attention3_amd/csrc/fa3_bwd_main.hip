@@ -315,10 +315,13 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 // so halving dKV only adds work: none from 0.54 to 0.75 (103 shapes against
 // bwd_main_kernel: the line above 0.93 on average and up to 1.08, none halved
 // 0.84, up to 1.05; nearer 0.5 the line halves a tile or two, as fast).
-// Full attention's jobs of a role are all alike, so all are halved or none;
-// whole jobs that fill less than two thirds of their last round of two
-// workgroups per CU also halve (B2 H12 S1792 D128: 672 jobs, -6 % whole, -11 %
-// halved).
+// Full attention's jobs of a role are all alike, so all are halved or none:
+// halved from 0.9 on, at D 64 with more than one head from 0.7 if S >= 512
+// (71 shapes of 0.7 .. 0.9, whole -> halved against bwd_main_kernel: S >= 1024
+// 1.00, up to 1.13 -> 0.84, up to 0.90; S 512 .. 1023 0.87 -> 0.74; shorter
+// ones 0.75 -> 0.69, but some up to 18 % slower halved).  D 128 with 1 to 4/3
+// rounds of two workgroups per CU, less than two thirds of the slots of two
+// rounds filled, also halves (B2 H12 S1792: 672 jobs, -6 % whole, -11 % halved).
 RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
     RegPlan r;
 #ifdef FA3_TIMELINE
@@ -357,7 +360,7 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
     } else {
         const double rounds = (double)p.batch * p.heads_kv * (chunks + group) * (qt / 2) /
                               (2 * kHeadSplitCus);
-        if (x > 0.9 ||
+        if (x > (d64 && heads > 1 && p.seqlen >= 512 ? 0.7 : 0.9) ||
             (p.head_dim == 128 && rounds > 1.0 && std::ceil(rounds) / rounds > 1.5))
             r.split_kv = 2;
     }

@@ -47,6 +47,12 @@ RULES = [
     (1, 5, 5, 8704, 64, True, "reg kv2 q2 c1"),          # (0.85)
     (2, 4, 4, 8064, 64, True, "reg h27/63 q1 c1"),       # (0.57)
     (6, 23, 23, 256, 64, True, "reg h2/2 q1 c1"),        # S < 512 (0.71)
+    # D 64 full, more than one head per dKV job: halved from 0.7 on
+    (2, 64, 4, 2816, 64, False, "reg kv2 q1 c1"),        # (0.83)
+    (2, 6, 2, 6144, 64, False, "reg kv2 q1 c1"),         # (0.76)
+    (3, 18, 6, 1664, 64, False, "reg kv1 q1 c1"),        # (0.63)
+    (1, 18, 18, 1408, 64, False, "reg kv1 q1 c1"),       # one head (0.74)
+    (13, 16, 8, 256, 64, False, "reg kv1 q1 c1"),        # S < 512 (0.70)
 ]
 
 
