@@ -316,12 +316,20 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 // bwd_main_kernel: the line above 0.93 on average and up to 1.08, none halved
 // 0.84, up to 1.05; nearer 0.5 the line halves a tile or two, as fast).
 // Full attention's jobs of a role are all alike, so all are halved or none:
-// halved from 0.9 on, at D 64 with more than one head from 0.7 if S >= 512
-// (71 shapes of 0.7 .. 0.9, whole -> halved against bwd_main_kernel: S >= 1024
-// 1.00, up to 1.13 -> 0.84, up to 0.90; S 512 .. 1023 0.87 -> 0.74; shorter
-// ones 0.75 -> 0.69, but some up to 18 % slower halved).  D 128 with 1 to 4/3
-// rounds of two workgroups per CU, less than two thirds of the slots of two
-// rounds filled, also halves (B2 H12 S1792: 672 jobs, -6 % whole, -11 % halved).
+// halved from 0.9 on, with these other lines (times against bwd_main_kernel):
+//   D 64, more than one head, S >= 512: from 0.7 on (71 shapes of 0.7 .. 0.9,
+//     whole -> halved: S >= 1024 1.00, up to 1.13 -> 0.84, up to 0.90; S 512 ..
+//     1023 0.87 -> 0.74; shorter 0.75 -> 0.69, but some 18 % slower halved);
+//   D 128, two heads: from 1.14 on, where the halved jobs are at most one per
+//     CU (above it whole 1.07, halved 0.82); of 0.9 .. 1.14 whole below S 1024
+//     (28 shapes, halved -> whole: 0.97, up to 1.11 -> 0.89, up to 1.02), and
+//     bwd_main_kernel from there on (whole 1.01 to 1.12, halved 1.02 to 1.14);
+//   D 128, four heads or more, S >= 1024: from 0.8 on (12 shapes of 0.8 .. 0.9,
+//     whole -> halved: 0.99, up to 1.03 -> 0.90);
+//   D 128: also with 1 to 4/3 rounds of two workgroups per CU, less than two
+//     thirds of the slots of two rounds filled (B2 H12 S1792: 672 jobs, -6 %
+//     whole, -11 % halved), but not with two heads and S >= 1024 (15 shapes,
+//     halved -> whole: 0.96, up to 1.02 -> 0.90).
 RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
     RegPlan r;
 #ifdef FA3_TIMELINE
@@ -360,8 +368,16 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
     } else {
         const double rounds = (double)p.batch * p.heads_kv * (chunks + group) * (qt / 2) /
                               (2 * kHeadSplitCus);
-        if (x > (d64 && heads > 1 && p.seqlen >= 512 ? 0.7 : 0.9) ||
-            (p.head_dim == 128 && rounds > 1.0 && std::ceil(rounds) / rounds > 1.5))
+        double most = 0.9;
+        if (d64 && heads > 1 && p.seqlen >= 512) most = 0.7;
+        if (!d64 && heads == 2) {
+            most = 1.14;
+            if (x > 0.9 && x <= most && p.seqlen >= 1024) r.on = false;
+        }
+        if (!d64 && heads > 3 && p.seqlen >= 1024) most = 0.8;
+        if (x > most ||
+            (!d64 && !(heads == 2 && p.seqlen >= 1024) && rounds > 1.0 &&
+             std::ceil(rounds) / rounds > 1.5))
             r.split_kv = 2;
     }
     return r;

@@ -53,6 +53,17 @@ RULES = [
     (3, 18, 6, 1664, 64, False, "reg kv1 q1 c1"),        # (0.63)
     (1, 18, 18, 1408, 64, False, "reg kv1 q1 c1"),       # one head (0.74)
     (13, 16, 8, 256, 64, False, "reg kv1 q1 c1"),        # S < 512 (0.70)
+    # D 128 full: halved with two heads per dKV job from 1.14 on, with four from 0.8
+    (8, 6, 3, 768, 128, False, "reg kv1 q1 c1"),         # two (1.02)
+    (2, 16, 1, 1152, 128, False, "main c8"),             # S >= 1024 (1.02)
+    (1, 34, 17, 1024, 128, False, "main c1"),            # (1.08)
+    (5, 4, 2, 2304, 128, False, "reg kv1 q1 c1"),        # 1.05 rounds (0.81)
+    (7, 14, 7, 512, 128, False, "reg kv2 q1 c1"),        # S < 1024 (0.75)
+    (1, 32, 16, 1024, 128, False, "reg kv2 q1 c1"),      # (1.14)
+    (1, 15, 5, 3712, 128, False, "reg kv2 q1 c1"),       # three (1.01)
+    (2, 16, 4, 2688, 128, False, "reg kv2 q1 c1"),       # four (0.87)
+    (1, 48, 8, 2944, 128, False, "reg kv1 q1 c1"),       # six (0.80)
+    (4, 264, 44, 128, 128, False, "reg kv1 q1 c1"),      # S < 1024 (0.83)
 ]
 
 
