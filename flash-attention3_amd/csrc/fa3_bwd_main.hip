@@ -384,7 +384,7 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
 }
 
 // The register-operand kernel's arguments, from a default-plan launch's.
-RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim) {
+RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim, bool causal) {
     RegArgs r{};
     r.q = a.q;
     r.k = a.k;
@@ -425,7 +425,7 @@ RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim) {
     r.scale = a.scale;
     r.n_groups = a.n_groups;
     r.halved = plan.halved;
-    set_reg_job_map(r, plan);
+    set_reg_job_map(r, plan, head_dim, causal);
     r.div_hkv = a.div_hkv;
     r.div_group = a.div_group;
     r.div_chunks = make_fastdiv(r.chunks);
@@ -445,8 +445,9 @@ void describe_launch(const BwdProblem& p, const WorkspacePlan& w, ShaoboFa3ExtPl
         r.seqlen = p.seqlen;
         r.group = group;
         r.chunks = chunks;
+        r.heads = group / chunks;
         r.n_groups = p.batch * p.heads_kv;
-        set_reg_job_map(r, reg);
+        set_reg_job_map(r, reg, p.head_dim, p.causal);
         o.jobs = r.n_groups * r.jobs_per_group;
         o.split_kv = reg.split_kv;
         o.halved = reg.halved;
@@ -578,7 +579,7 @@ hipError_t launch_backward(const BwdProblem& p, const BwdTensors& t, void* works
     }
     const RegPlan reg = reg_plan(p, plan);
     if (reg.on) {
-        const RegArgs r = reg_args(a, reg, p.head_dim);
+        const RegArgs r = reg_args(a, reg, p.head_dim, p.causal);
         if (g_debug_kernels.load())
             launch_reg_race_check(r, reg, p.head_dim, p.causal, p.bf16, t.stream);
         else launch_reg_kernel<false>(r, reg, p.head_dim, p.causal, p.bf16, t.stream);

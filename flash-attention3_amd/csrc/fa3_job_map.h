@@ -29,15 +29,21 @@ inline constexpr int kInterleaveJobsPerCu = 8;
 inline constexpr double kInterleaveTail = 2.0;
 inline constexpr int kInterleaveSpan = 4;
 
+// The smallest split of the groups into parts that deals whole parts to the
+// XCDs: n_groups * parts % 8 == 0.
+inline int xcd_split(int n_groups) {
+    int gcd8 = 8;
+    while (n_groups % gcd8 != 0) gcd8 >>= 1;
+    return 8 / gcd8;
+}
+
 // XCD-aware job map of a.n_groups groups of a.jobs_per_group jobs, an XCD's
 // groups one after another or interleaved (A: FusedArgs, or RegArgs of
-// fa3_bwd_reg_kernel.h).
+// fa3_bwd_reg_kernel.h); by_parts false: without the XCDs' parts.
 template <typename A, typename Choose>
-inline void set_job_map_with(A& a, Choose&& interleave_of) {
-    int gcd8 = 8;
-    while (a.n_groups % gcd8 != 0) gcd8 >>= 1;
-    const int parts = 8 / gcd8;  // smallest split with n_groups * parts % 8 == 0
-    const bool fits = a.jobs_per_group % parts == 0;
+inline void set_job_map_with(A& a, Choose&& interleave_of, bool by_parts = true) {
+    const int parts = xcd_split(a.n_groups);
+    const bool fits = by_parts && a.jobs_per_group % parts == 0;
     a.xcd_parts = fits ? parts : 0;
     a.xcd_vgroups = fits ? a.n_groups * parts / 8 : 0;
     // the groups an XCD's virtual groups belong to (one more where its
@@ -64,19 +70,32 @@ inline void set_job_map(FusedArgs& a, double longest = 0.0, double share = 1.0, 
     });
 }
 
-// The map of bwd_reg_kernel's launches (seqlen, group, chunks and n_groups
-// set).  Always position by position across an XCD's groups, longest jobs
-// first: the hardware deals the jobs out in this order, and with small
+// The map of bwd_reg_kernel's launches (seqlen, group, chunks, heads and
+// n_groups set).  Always position by position across an XCD's groups, longest
+// jobs first: the hardware deals the jobs out in this order, and with small
 // workgroups a late long job costs more than the L2 gains from one group at a
 // time (B2 Hq32 Hkv8 S4096 D128 causal 1 029 -> 866 us, B4 H16 S1024 95.9 ->
 // 71.4, B4 H16 S2048 267.8 -> 240.7, B1 H16 S8192 783 -> 771; full attention,
 // B2 H12 S1664 D64 70.9 -> 63.8, B2 H16 S8192 D64 equal though five times the
 // algorithmic bytes are fetched).
-inline void set_reg_job_map(RegArgs& r, const RegPlan& plan) {
+// Groups cut into parts of one job have no order inside an XCD: all roles and
+// lengths come mixed, group after group.  With three heads per dKV job or more,
+// which is then several times as long as a dQ job, the positions run across
+// all groups instead (106 shapes of S 128 and 256, parts -> across against
+// bwd_main_kernel: D 128 0.93, up to 1.10 -> 0.81, up to 0.85; D 64 0.82 -> 0.68);
+// so they do at D 128 causal with one head and parts of one or two jobs, S >=
+// 512 (67 shapes: 0.95, up to 1.05 -> 0.87, up to 0.91).  Elsewhere the parts' L2
+// gain is worth as much or more (across 0.9 to 1.25 of their time).
+inline void set_reg_job_map(RegArgs& r, const RegPlan& plan, int head_dim, bool causal) {
     r.jobs_per_group =
         r.seqlen / 128 * (std::max(plan.split_kv, 1) * r.chunks + plan.split_q * r.group) +
         plan.halved * r.chunks;
-    set_job_map_with(r, [](int) { return true; });
+    const int parts = xcd_split(r.n_groups);
+    const int most = r.heads > 2 ? 1
+                     : r.heads == 1 && head_dim == 128 && causal && r.seqlen >= 512 ? 2
+                                                                                     : 0;
+    set_job_map_with(r, [](int) { return true; },
+                     parts < 4 || r.jobs_per_group > most * parts);
 }
 
 }  // namespace fa3

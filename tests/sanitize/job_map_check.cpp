@@ -136,7 +136,10 @@ int main() {
                         plan.split_kv = c.kv;
                         plan.split_q = c.q;
                         plan.halved = c.halved;
-                        fa3::set_reg_job_map(r, plan);
+                        r.heads = group / chunks;
+                        const bool causal = c.kv == 0;
+                        const int head_dim = c.q == 2 || chunks % 2 == 0 ? 64 : 128;
+                        fa3::set_reg_job_map(r, plan, head_dim, causal);
                         if (r.jobs_per_group != chunks * c.dkv + group * c.dq) {
                             std::printf("register kernel: %d jobs per group, want %d\n",
                                         r.jobs_per_group, chunks * c.dkv + group * c.dq);

@@ -31,6 +31,8 @@ CASES = [
     (1, 20, 5, 768, 64, False, "bf16", True, None, "reg kv2 q2 c4"),       # both halved, a chunk per head (1.22)
     (2, 12, 12, 1792, 128, False, "bf16", False, None, "reg kv2 q1 c1"),   # 1.3 rounds of workgroups (0.44)
     (3, 21, 21, 384, 64, True, "fp16", False, None, "reg kv2 q2 c1"),      # both roles halved, D 64 (1.16)
+    (11, 57, 19, 256, 128, True, "bf16", False, None, "reg h0/2 q1 c1"),   # parts of one job: dealt across the groups (0.47)
+    (3, 87, 29, 256, 64, False, "fp16", True, None, "reg kv1 q1 c1"),      # likewise, D 64, full (0.84)
     (3, 19, 19, 128, 64, True, "bf16", False, 1.0, "main c1"),             # few jobs (2.57)
 ]
 

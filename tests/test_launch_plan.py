@@ -72,6 +72,27 @@ def test_rule(B, Hq, Hkv, S, D, causal, plan):
     assert launch_plan(B, Hq, Hkv, S, D, causal) == plan
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,jobs,parts", [
+    # jobs per group; the parts they are dealt to the XCDs in, 0: across all groups
+    (11, 57, 19, 256, 128, True, 8, 0),    # eight parts would hold one job each
+    (3, 33, 33, 512, 128, True, 8, 0),     # one head
+    (3, 19, 19, 1024, 128, True, 16, 0),   # D 128 causal: two jobs each
+    (5, 50, 50, 256, 128, True, 4, 4),     # S < 512
+    (3, 19, 19, 1536, 128, True, 24, 8),   # three
+    (9, 90, 30, 128, 128, False, 4, 0),    # four parts of one job, three heads
+    (3, 87, 29, 256, 64, False, 8, 0),     # three heads
+    (9, 87, 29, 512, 64, False, 16, 8),    # two jobs each
+    (5, 45, 15, 512, 128, False, 16, 8),
+    (3, 53, 53, 512, 64, False, 8, 8),     # one head: the parts stay
+    (8, 25, 25, 128, 128, True, 2, 1),     # aligned group count
+    (2, 49, 49, 384, 128, True, 6, 0),     # four parts do not divide six jobs
+])
+def test_job_map_parts(B, Hq, Hkv, S, D, causal, jobs, parts):
+    p = F.plan_of(F.make_params(batch=B, seqlen=S, heads_q=Hq, heads_kv=Hkv, head_dim=D,
+                                causal=causal))
+    assert (p.kernel, p.jobs, p.xcd_parts) == (F.KERNEL_REG, jobs * B * Hkv, parts)
+
+
 @pytest.mark.parametrize("row", CASES, ids=lambda r: "-".join(map(str, r[:6])))
 def test_reg_kernel_rows_run_what_they_say(row):
     assert launch_plan(*row[:6]) == row[-1]
