@@ -25,6 +25,7 @@ import importlib.machinery
 import importlib.util
 import math
 import os
+import warnings
 from typing import Optional, Tuple
 
 import torch
@@ -51,18 +52,23 @@ _NATIVE = None
 
 def _native():
     """The native body (csrc/fa3_torch_op.cpp), or False where it has not been
-    built (`make -C flash-attention3_amd torch`): then the same body runs in
-    Python through ctypes."""
+    built (`make -C flash-attention3_amd torch`) or does not load, being built
+    for another Python, torch or library (said once, in a warning): then the
+    same body runs in Python through ctypes."""
     global _NATIVE
     if _NATIVE is None:
+        body = False
         if os.path.exists(_NATIVE_PATH):
             loader = importlib.machinery.ExtensionFileLoader("_fa3_torch", _NATIVE_PATH)
             spec = importlib.util.spec_from_loader("_fa3_torch", loader)
-            mod = importlib.util.module_from_spec(spec)
-            loader.exec_module(mod)
-            _NATIVE = mod.backward
-        else:
-            _NATIVE = False
+            try:
+                mod = importlib.util.module_from_spec(spec)
+                loader.exec_module(mod)
+                body = mod.backward
+            except ImportError as e:
+                warnings.warn(f"{_NATIVE_PATH} does not load, the op's body runs in Python: {e}",
+                              RuntimeWarning, stacklevel=2)
+        _NATIVE = body
     return _NATIVE
 
 

@@ -1,12 +1,14 @@
 """PyTorch custom-op binding (flash-attention3_amd/shaobo_fa3_torch.py), host
 side: registration, the fake implementation's shapes, argument checks.  The
 GPU behaviour is in test_gpu_torch_op.py."""
+import warnings
+
 import pytest
 
 torch = pytest.importorskip("torch")
 from torch._subclasses.fake_tensor import FakeTensorMode  # noqa: E402
 
-import shaobo_fa3_torch  # noqa: E402,F401  (registers the op)
+import shaobo_fa3_torch as T  # noqa: E402  (registers the op)
 
 
 def tensors(B=2, Hq=4, Hkv=2, S=256, D=128, dtype=torch.float16):
@@ -55,3 +57,22 @@ def test_fake_rejects_bad_arguments(bad):
             q = q.transpose(1, 2)
         with pytest.raises(ValueError):
             torch.ops.shaobo_fa3.flash_attn_backward(dout, q, k, v, out, lse, True, None, False)
+
+
+def test_native_body_that_does_not_load_falls_back(tmp_path, monkeypatch):
+    """A _fa3_torch.so built for another Python, torch or library leaves the op
+    its Python body, with one warning that names the reason."""
+    bad = tmp_path / "_fa3_torch.so"
+    bad.write_bytes(b"not a shared object")
+    monkeypatch.setattr(T, "_NATIVE", None)
+    monkeypatch.setattr(T, "_NATIVE_PATH", str(bad))
+    with pytest.warns(RuntimeWarning, match="_fa3_torch.so"):
+        assert T._native() is False
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert T._native() is False
+    monkeypatch.setattr(T, "_NATIVE", None)
+    monkeypatch.setattr(T, "_NATIVE_PATH", str(tmp_path / "absent.so"))
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert T._native() is False
