@@ -1,6 +1,10 @@
 """PyTorch custom-op binding (flash-attention3_amd/shaobo_fa3_torch.py), host
 side: registration, the fake implementation's shapes, argument checks.  The
 GPU behaviour is in test_gpu_torch_op.py."""
+import os
+import shutil
+import subprocess
+import sys
 import warnings
 
 import pytest
@@ -76,3 +80,22 @@ def test_native_body_that_does_not_load_falls_back(tmp_path, monkeypatch):
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert T._native() is False
+
+
+@pytest.mark.skipif(shutil.which("make") is None, reason="no make")
+def test_build_keeps_the_native_body_in_step(monkeypatch):
+    """`make all` rebuilds an op body that is there, and the body is built for
+    the interpreter that build() runs in."""
+    if not os.path.exists(T._NATIVE_PATH):
+        pytest.skip("lib/_fa3_torch.so is not built")
+    pkg = os.path.dirname(os.path.dirname(T._NATIVE_PATH))
+    dry = lambda *a: subprocess.run(["make", "-n", "-B", "-C", pkg, *a], text=True,  # noqa: E731
+                                    capture_output=True, check=True).stdout
+    assert "_fa3_torch.so" in dry("all")
+    monkeypatch.syspath_prepend(os.path.dirname(pkg))
+    import __graft_entry__ as entry
+    calls = []
+    monkeypatch.setattr(entry, "_make", lambda path, *targets: calls.append((path, targets)))
+    entry.build()
+    targets = next(t for p, t in calls if p == pkg)
+    assert f"{sys.executable} -c" in dry(*targets)
