@@ -340,7 +340,7 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
 #ifdef FA3_TIMELINE
     return r;  // the stamps are bwd_main_kernel's
 #endif
-    if (w.bal_m > 0) return r;
+    if (w.bal_m > 0 || p.out_f32) return r;  // (its outputs are 16-bit)
     const int group = p.heads_q / p.heads_kv, chunks = std::max(w.hs_chunks, 1);
     const int heads = group / chunks, qt = p.seqlen / 64;  // (qt even)
     const double units = p.causal ? 0.25 * qt * (qt + 2.0) : 0.5 * qt * qt;
@@ -404,7 +404,7 @@ RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim, bool causal) {
     r.nlse2 = a.nlse2;
     r.ndelta = a.ndelta;
     r.dq = a.dq;
-    r.dq_f32 = a.out_f32;
+    r.dq_f32 = 0;
     r.q_rs = a.q_rs;
     r.q_hs = a.q_hs;
     r.kv_rs = a.kv_rs;
@@ -427,7 +427,7 @@ RegArgs reg_args(const FusedArgs& a, RegPlan plan, int head_dim, bool causal) {
         r.heads = a.group;
         r.dk = a.dk;
         r.dv = a.dv;
-        r.dkv_f32 = a.out_f32;
+        r.dkv_f32 = 0;
         r.o_rs = a.kv_rs;
         r.o_hs = a.kv_hs;
         r.o_heads = a.heads_kv;

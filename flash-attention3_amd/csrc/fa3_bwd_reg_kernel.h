@@ -65,6 +65,9 @@ struct RegArgs {
     void* dq;
     void* dk;  // the outputs, or the head-split plan's fp32 contributions
     void* dv;
+    // fp32 instead of 16-bit stores: dkv_f32 with the head split, dq_f32 never
+    // (0) -- the branch stays because without it the compiler spills 9 vector
+    // registers of the D 128 full-attention kernels.
     int dq_f32, dkv_f32;
     int q_rs, q_hs, kv_rs, kv_hs;  // as in FusedArgs
     int o_rs, o_hs, o_heads;       // dK / dV: row stride, head stride, heads
