@@ -14,7 +14,7 @@ import pytest
 
 import fa3_oracle as O
 import shaobo_fa3 as F
-from gpu_util import check, dev, log, run_v2
+from gpu_util import check, dev, launch_plan, log, run_v2
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -48,7 +48,7 @@ CASES = [
     (1, 9, 9, 2048, 64, True),    # 576 jobs: causal, one head per group, default plan
     (1, 4, 2, 1024, 128, True),   # head-split plan: G = 2, one head per chunk
     (1, 8, 1, 1024, 128, True),   # head-split plan: MQA, G = 8, one head per chunk
-    (1, 16, 2, 2048, 64, False),  # head-split plan: full, D = 64, two heads per chunk
+    (1, 16, 2, 2048, 64, False),  # head split (bwd_reg_kernel): full, D = 64, two heads per chunk
     (1, 12, 12, 512, 128, True),  # split plan over 12 groups: XCD-interleaved job map
     (1, 12, 12, 1024, 128, True), # 384 jobs: one job per workgroup, interleaved
     (3, 8, 2, 512, 64, False),    # 6 groups, head split, one job per workgroup, interleaved
@@ -321,20 +321,28 @@ def test_dot_do_o_component(lse_mode):
         np.testing.assert_allclose(pk[:, 1], 1.0 / g["scores_sum"].ravel(), rtol=1e-6)
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal", [
-    (2, 32, 8, 4096, 128, True),    # P4 GQA
-    (2, 16, 16, 8192, 64, False),   # P5
-    (1, 32, 1, 4096, 128, True),    # MQA at batch 1: head-split plan, 4 heads per chunk
-    (1, 19, 19, 4096, 64, True),    # 19 groups, 3 per XCD, 9.5 jobs per CU: tail interleaving
-])
-def test_full_size_configs(B, Hq, Hkv, S, D, causal):
-    """The whole P4 / P5 backward against the oracle (forward and backward
+FULL_SIZE = [
+    # B, Hq, Hkv, S, D, causal, plan (gpu_util.launch_plan)
+    (2, 32, 8, 4096, 128, True, "reg h4/32 q1 c1"),    # P4 GQA
+    (2, 16, 16, 8192, 64, False, "reg kv1 q1 c1"),     # P5
+    (1, 32, 1, 4096, 128, True, "reg h18/32 q1 c8"),   # MQA at batch 1: head split, 4 heads per chunk
+    (1, 19, 19, 4096, 64, True, "reg h10/32 q1 c1"),   # 19 groups
+    # bwd_main_kernel past 2048 jobs (eight per CU), persistent:
+    (5, 20, 4, 1280, 128, True, "main c1"),            # 2400 jobs, 5 virtual groups per XCD: tail interleaving
+    (2, 16, 4, 3456, 128, True, "main c1"),            # 2160 jobs, one group per XCD after another
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,plan", FULL_SIZE)
+def test_full_size_configs(B, Hq, Hkv, S, D, causal, plan):
+    """The whole P4 / P5 backward, and others of many jobs, against the oracle (forward and backward
     on the CPU, about 10 s with 16 threads), checked per (batch, kv-head)
     group -- dK / dV of the group's KV head, dQ / delta of its query heads,
     each against its own max|ref| -- so a job-map error confined to some
     groups cannot hide behind the others' magnitudes (the reference's gate
     compares whole tensors: src/full_bwd_correctness.cpp:471-500)."""
-    log(f"[case] full-size B={B} Hq={Hq} Hkv={Hkv} S={S} D={D} causal={causal}")
+    log(f"[case] full-size B={B} Hq={Hq} Hkv={Hkv} S={S} D={D} causal={causal}: {plan}")
+    assert launch_plan(B, Hq, Hkv, S, D, causal) == plan
     g = O.golden(B, Hq, Hkv, S, D, causal)
     res = run_v2(g, torch)
     assert res["status"] == F.SUCCESS
@@ -359,23 +367,29 @@ def check_per_group(res, g):
     log({"worst group": {k: round(v, 6) for k, v in worst.items()}})
 
 
-@pytest.mark.parametrize("hq,hkv", [
-    (16, 8),  # 1536 jobs, one dKV job per KV head
-    (8, 2),   # 1024 jobs, head-split plan (a merged dKV job, 256 steps, would
-              # outlast a CU's share of the work)
-])
+MANY_JOBS = [
+    # Hq, Hkv, S, plan, at B1 D128 causal
+    (16, 8, 4096, "reg h18/32 q1 c1"),   # bwd_reg_kernel, one dKV job per KV head
+    (8, 2, 4096, "main c4"),             # bwd_main_kernel, persistent (1024 jobs), head split
+    (4, 2, 8192, "main c1"),             # ... (768 jobs), one dKV job per KV head
+]
+
+
+@pytest.mark.parametrize("hq,hkv,s,plan", MANY_JOBS)
 @pytest.mark.parametrize("dtype,layout,scale", [
-    ("bf16", "bhsd", None),   # bf16 instantiation of the persistent plan
-    ("fp16", "bshd", None),   # BSHD strides in the persistent job loop
-    ("fp16", "bhsd", 1.0),    # scale 1: c = log2(e) > 1, the unscaled instantiation
+    ("bf16", "bhsd", None),   # bf16 instantiations
+    ("fp16", "bshd", None),   # BSHD strides (in the persistent job loop)
+    ("fp16", "bhsd", 1.0),    # scale 1: c = log2(e) > 1, bwd_main_kernel's unscaled instantiation
 ])
-def test_persistent_plan_variants(dtype, layout, scale, hq, hkv):
-    """The persistent default plan (more than two jobs per CU) at B1 S4096
-    D128 causal, GQA, in the instantiations the BASELINE configs do not reach
-    -- bf16, BSHD, unscaled resident operands -- against the oracle, per
-    (batch, kv-head) group; BSHD also bit-equal to BHSD."""
-    log(f"[case] persistent plan {dtype} {layout} scale={scale} B1 Hq{hq} Hkv{hkv} S4096 D128 causal")
-    g = O.golden(1, hq, hkv, 4096, 128, True, scale=scale, dtype=dtype)
+def test_persistent_plan_variants(dtype, layout, scale, hq, hkv, s, plan):
+    """Launches of many jobs at B1 D128 causal, GQA -- bwd_main_kernel's
+    persistent plan, and bwd_reg_kernel for the first -- in the instantiations
+    that P1 .. P5 do not reach (bf16, BSHD, unscaled resident operands),
+    against the oracle, per (batch, kv-head) group; BSHD also bit-equal to
+    BHSD."""
+    log(f"[case] {plan}: {dtype} {layout} scale={scale} B1 Hq{hq} Hkv{hkv} S{s} D128 causal")
+    assert launch_plan(1, hq, hkv, s, 128, True) == plan
+    g = O.golden(1, hq, hkv, s, 128, True, scale=scale, dtype=dtype)
     res = run_v2(g, torch, bshd=layout == "bshd")
     assert res["status"] == F.SUCCESS, F.status_name(res["status"])
     check_per_group(res, g)

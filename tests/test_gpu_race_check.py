@@ -1,9 +1,10 @@
 """GPU race checks (the counterpart of the reference's stress run that caught
-races in its kernel, reference source_status.md:608-612): the main kernel's
-race-check instantiation -- the same arithmetic, every job started on an LDS
+races in its kernel, reference source_status.md:608-612): the main kernels'
+race-check instantiations -- the same arithmetic, every job started on an LDS
 poisoned with NaN bytes, a full wait and a barrier after every LDS phase of
-the pipeline -- must give the fast kernel's outputs bit for bit, under the
-split plan, the persistent plan and the one-job-per-workgroup plan.  A read
+the pipeline -- must give the fast kernels' outputs bit for bit, in
+bwd_main_kernel's split, persistent and one-job-per-workgroup plans and in
+bwd_reg_kernel (more of it in test_gpu_reg_kernel.py).  A read
 of LDS that a job did not write shows up as NaN (and fails the oracle
 check), a race between the fast kernel's waves as a bitwise difference.
 Also here: the split-wait give-up reported to unsynchronised callers, and
@@ -15,7 +16,7 @@ import pytest
 
 import fa3_oracle as O
 import shaobo_fa3 as F
-from gpu_util import check, log, run_v2
+from gpu_util import check, launch_plan, log, run_v2
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -38,24 +39,31 @@ def race_checked(g, **kw):
 
 
 RACE_CASES = [
-    # B, Hq, Hkv, S, D, causal, dtype, plan
-    (1, 1, 1, 128, 128, True, "fp16"),     # P1: one job per workgroup
-    (1, 1, 1, 1024, 128, True, "fp16"),    # P2: split plan
-    (1, 4, 4, 2048, 128, True, "fp16"),    # P3: split plan (the headline)
-    (1, 9, 9, 2048, 64, True, "fp16"),     # 576 jobs: persistent plan, D 64
-    (4, 16, 8, 1024, 128, True, "fp16"),   # 1536 jobs: persistent plan, GQA, D 128
-    (2, 16, 4, 1024, 128, True, "fp16"),   # 1024 jobs: head-split plan
-    (1, 16, 2, 2048, 64, False, "fp16"),   # head-split plan, two query heads per chunk
-    (2, 16, 4, 2048, 128, True, "fp16"),   # 1280 jobs: five per workgroup
-    (2, 8, 8, 1024, 64, False, "fp16"),    # 512 jobs: one job per workgroup, full attention
-    (3, 8, 8, 1024, 64, False, "fp16"),    # 768 jobs: persistent plan, full attention
-    (1, 2, 2, 512, 128, True, "bf16"),     # bf16, split plan
+    # B, Hq, Hkv, S, D, causal, dtype, plan (gpu_util.launch_plan)
+    (1, 1, 1, 128, 128, True, "fp16", "main c1"),           # P1: one job per workgroup
+    (1, 1, 1, 1024, 128, True, "fp16", "split"),            # P2
+    (1, 4, 4, 2048, 128, True, "fp16", "split"),            # P3 (the headline)
+    (1, 9, 9, 2048, 64, True, "fp16", "main c1"),           # 576 jobs: persistent, D 64
+    (4, 16, 8, 1024, 128, True, "fp16", "reg h5/8 q1 c1"),  # GQA, D 128
+    (2, 16, 4, 1024, 128, True, "fp16", "reg h5/8 q1 c4"),  # head split
+    (1, 16, 2, 2048, 64, False, "fp16", "reg kv2 q1 c4"),   # head split, two query heads per chunk
+    (2, 16, 4, 2048, 128, True, "fp16", "main c1"),         # 1280 jobs: five per workgroup
+    (2, 8, 8, 1024, 64, False, "fp16", "reg kv2 q2 c1"),    # full attention
+    (3, 8, 8, 1024, 64, False, "fp16", "reg kv1 q1 c1"),
+    (1, 2, 2, 512, 128, True, "bf16", "split"),             # bf16
+    # bwd_main_kernel: head split and full attention
+    (2, 9, 3, 1536, 128, True, "fp16", "main c3"),          # 864 jobs: persistent head split
+    (1, 20, 5, 768, 128, False, "bf16", "main c4"),         # 480 jobs: head split, full
+    (2, 6, 2, 1024, 64, False, "fp16", "main c3"),          # ... D 64
+    (2, 8, 8, 1024, 128, False, "fp16", "main c1"),         # 512 jobs: one per workgroup, full
+    (3, 5, 5, 1536, 128, False, "fp16", "main c1"),         # 720 jobs: persistent, full
 ]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,dtype", RACE_CASES)
-def test_race_check_kernel_is_bit_equal(B, Hq, Hkv, S, D, causal, dtype):
-    log(f"[case] race check B={B} Hq={Hq} Hkv={Hkv} S={S} D={D} causal={causal} {dtype}")
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,dtype,plan", RACE_CASES)
+def test_race_check_kernel_is_bit_equal(B, Hq, Hkv, S, D, causal, dtype, plan):
+    log(f"[case] race check B={B} Hq={Hq} Hkv={Hkv} S={S} D={D} causal={causal} {dtype}: {plan}")
+    assert launch_plan(B, Hq, Hkv, S, D, causal) == plan
     g = O.golden(B, Hq, Hkv, S, D, causal, dtype=dtype)
     fast = run_v2(g, torch)
     slow = race_checked(g)

@@ -1,8 +1,8 @@
 """The register-operand main kernel (bwd_reg_kernel) at the edges of the
 shapes that reach it: a single 128-row tile, odd tile counts, group counts
-without XCD-aligned parts, each way of cutting the jobs (whole, dKV halved,
-both halved), fp32 head-split contributions, bf16, BSHD and a scale above
-ln 2.  Each case against the CPU oracle under the bar of gpu_util.check,
+without XCD-aligned parts, each way of cutting the jobs at each head dim and
+mask (whole, some or all dKV halved, both roles halved), fp32 head-split
+contributions, bf16, BSHD and a scale above ln 2.  Each case against the CPU oracle under the bar of gpu_util.check,
 bitwise repeatable, and bit for bit equal to its race-check instantiation
 (every job on an LDS of NaN bytes, a full wait and a barrier around every
 phase)."""
@@ -31,6 +31,12 @@ CASES = [
     (1, 20, 5, 768, 64, False, "bf16", True, None, "reg kv2 q2 c4"),       # both halved, a chunk per head (1.22)
     (2, 12, 12, 1792, 128, False, "bf16", False, None, "reg kv2 q1 c1"),   # 1.3 rounds of workgroups (0.44)
     (3, 21, 21, 384, 64, True, "fp16", False, None, "reg kv2 q2 c1"),      # both roles halved, D 64 (1.16)
+    (3, 43, 43, 384, 128, False, "fp16", False, None, "reg kv1 q1 c1"),    # full, whole jobs (0.38)
+    (4, 64, 32, 512, 128, False, "bf16", True, None, "reg kv1 q1 c1"),     # ... G 2, BSHD (0.29)
+    (5, 64, 32, 512, 128, True, "fp16", False, None, "reg h0/4 q1 c1"),    # causal, whole, G 2 (0.37)
+    (7, 32, 32, 512, 64, True, "fp16", False, None, "reg h0/4 q1 c1"),     # ... D 64 (0.26)
+    (4, 40, 20, 1408, 64, True, "bf16", True, None, "reg h0/11 q1 c1"),    # ... G 2, BSHD (0.30)
+    (4, 32, 16, 512, 64, True, "bf16", True, None, "reg h3/4 q1 c1"),      # some halved, D 64, G 2 (0.91)
     (11, 57, 19, 256, 128, True, "bf16", False, None, "reg h0/2 q1 c1"),   # parts of one job: dealt across the groups (0.47)
     (3, 87, 29, 256, 64, False, "fp16", True, None, "reg kv1 q1 c1"),      # likewise, D 64, full (0.84)
     (3, 19, 19, 128, 64, True, "bf16", False, 1.0, "main c1"),             # few jobs (2.57)

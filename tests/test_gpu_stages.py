@@ -10,24 +10,26 @@ import ctypes
 import pytest
 
 import shaobo_fa3 as F
-from gpu_util import log
+from gpu_util import launch_plan, log
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # (B, Hq, Hkv, S, D, causal)   plan
-    (1, 4, 4, 2048, 128, True),    # split plan (P3)
-    (1, 5, 5, 4096, 128, False),   # persistent: 5 heads x 64 tiles x 2 roles = 640 jobs
-    (1, 4, 4, 4096, 128, False),   # 512 jobs: one job per workgroup
-    (2, 8, 2, 2048, 64, True),     # persistent, GQA, D 64 (B 2 x Hkv 2 x 32 x 5 = 640 jobs)
+    # B, Hq, Hkv, S, D, causal, plan (gpu_util.launch_plan)
+    (1, 4, 4, 2048, 128, True, "split"),           # P3
+    (1, 5, 5, 4096, 128, False, "main c1"),        # persistent: 5 heads x 64 tiles x 2 roles = 640 jobs
+    (1, 4, 4, 4096, 128, False, "main c1"),        # 512 jobs: one job per workgroup
+    (2, 8, 2, 2048, 64, True, "reg kv2 q2 c4"),    # bwd_reg_kernel, head split
+    (2, 8, 4, 2048, 64, True, "main c1"),          # persistent, GQA, D 64 (B 2 x Hkv 4 x 32 x 3 = 768 jobs)
 ]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal", CASES)
-def test_stages_match_full_call(B, Hq, Hkv, S, D, causal):
-    log(f"stages B{B} Hq{Hq} Hkv{Hkv} S{S} D{D} causal={causal}")
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,causal,plan", CASES)
+def test_stages_match_full_call(B, Hq, Hkv, S, D, causal, plan):
+    log(f"stages B{B} Hq{Hq} Hkv{Hkv} S{S} D{D} causal={causal}: {plan}")
     lib = F.load()
+    assert launch_plan(B, Hq, Hkv, S, D, causal) == plan
     gen = torch.Generator(device="cuda").manual_seed(7)
     mk = lambda h: torch.randn((B, h, S, D), generator=gen, device="cuda").half()  # noqa: E731
     q, k, v, do, out = mk(Hq), mk(Hkv), mk(Hkv), mk(Hq), mk(Hq)

@@ -6,7 +6,15 @@ import pytest
 
 import shaobo_fa3 as F
 from gpu_util import launch_plan
-from test_gpu_reg_kernel import CASES
+import test_gpu_parity
+import test_gpu_race_check
+import test_gpu_reg_kernel
+import test_gpu_stages
+
+CASES = [r[:6] + r[-1:] for rows in (test_gpu_reg_kernel.CASES, test_gpu_race_check.RACE_CASES,
+                                     test_gpu_stages.CASES, test_gpu_parity.FULL_SIZE)
+         for r in rows]
+CASES += [(1, hq, hkv, s, 128, True, plan) for hq, hkv, s, plan in test_gpu_parity.MANY_JOBS]
 
 
 def test_plan_arguments():
@@ -100,5 +108,5 @@ def test_job_map_parts(B, Hq, Hkv, S, D, causal, jobs, parts):
 
 
 @pytest.mark.parametrize("row", CASES, ids=lambda r: "-".join(map(str, r[:6])))
-def test_reg_kernel_rows_run_what_they_say(row):
+def test_gpu_rows_run_what_they_say(row):
     assert launch_plan(*row[:6]) == row[-1]

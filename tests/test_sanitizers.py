@@ -7,7 +7,7 @@ host-computed fast division against / under UBSan (tests/sanitize/fastdiv_check.
 and the split plan's planner against its invariants under ASan + UBSan
 (tests/sanitize/split_plan_check.cpp), the stream entries' stream-device
 rule under UBSan (tests/sanitize/launch_device_check.cpp), and the main
-kernel's job map -- a bijection onto (group, position), parts pinned to one
+kernels' job maps -- a bijection onto (group, position), parts pinned to one
 XCD, longest jobs first when interleaved -- under UBSan
 (tests/sanitize/job_map_check.cpp).  Built by
 tests/sanitize/Makefile."""
