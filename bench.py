@@ -1,10 +1,9 @@
 """Benchmark of the FA3 backward (shaobo_fa3_bwd_v2) on one MI355X.
 
 A step is one full backward through the C ABI over resident fp16 inputs at
-the headline shape B=1, H=4, S=2048, D=128, causal (BASELINE.json
-configs[2]): the delta preprocess and the main kernel, two launches on the
-null stream.  The timed region is `steps` back-to-back shaobo_fa3_bwd_v2
-calls between two HIP events.  Per-kernel durations, back to back: the main
+the headline shape B=1, H=4, S=2048, D=128, causal: the delta preprocess and
+the main kernel, two launches on the null stream.  The timed region is `steps`
+back-to-back shaobo_fa3_bwd_v2 calls between two HIP events.  Per-kernel durations, back to back: the main
 kernel alone over as many back-to-back launches between two events
 (shaobo_fa3_ext_bwd_v2_stages with the main-kernel stage, on the workspace
 the timed calls prepared), and the preprocess as the step minus that -- its
@@ -20,7 +19,7 @@ line: TFLOP/s from FLOPs = 10*B*H*S^2*D*0.5, ms per backward, % of fp16 dense
 MFMA peak, the main kernel's (MFMA) and the preprocess's (HBM) rooflines,
 and the CPU oracle timed on the host as the reported CPU baseline.
 
---all measures every BASELINE config (P1-P5) in one run and prints one JSON
+--all measures every configuration P1-P5 in one run and prints one JSON
 line per config (GPU ms per backward, TFLOP/s, % of peak, the main kernel's
 time, and the CPU oracle's backward of the whole config on the host, with
 the threads it used and the host's core count), then a markdown table of
@@ -119,12 +118,6 @@ class Hip:
         assert self.lib.hipDeviceSynchronize() == 0
 
 
-# The kernel behind the main stage (key "bwd_main_kernel" of the times) of
-# each configuration; another --shape runs either of the two.
-MAIN_KERNEL = {"P1": "bwd_main_kernel", "P2": "bwd_main_kernel", "P3": "bwd_main_kernel",
-               "P4": "bwd_reg_kernel", "P5": "bwd_reg_kernel"}
-
-
 def load_traffic(config):
     """HBM bytes per launch of the main kernel, measured with rocprofv3
     FETCH_SIZE / WRITE_SIZE and scaled by a copy kernel of known size
@@ -153,8 +146,8 @@ def host_cores():
         return os.cpu_count() or 1
 
 
-# The oracle runs on at most this many threads: a GPU box gives one GPU a
-# 16-core share of its host, whatever the affinity mask shows.
+# The oracle runs on at most this many threads: one GPU's share of an 8-GPU
+# host's cores, whatever the affinity mask shows.
 CPU_SHARE_PER_GPU = 16
 
 
@@ -217,8 +210,8 @@ def cpu_baseline(cfg, budget_s):
                         "tflops": round(flops(b1, hq1, s1, d1, c1) / dt / 1e12, 6)}
     return {"value": round(f / sec / 1e12, 6), "unit": "TFLOP/s", "cores": threads,
             "host_cores": host_cores(),
-            "threads_note": f"threads = min(host cores, {CPU_SHARE_PER_GPU}): the GPU box's "
-                            "CPU share per GPU",
+            "threads_note": f"threads = min(host cores, {CPU_SHARE_PER_GPU}): one GPU's share "
+                            "of the host's cores",
             "kind": "port",
             "sample": f"oracle fp32 backward of {sample_heads} of {B * Hq} query heads "
                       f"(S={S}, D={D}, causal={causal}), {runs} runs, {sec * 1e3:.1f} ms each",
@@ -371,7 +364,9 @@ def measure(torch, lib, F, hip, name, steps, warmup, deterministic, dtype="fp16"
         "kernels_ms_marked": {"preprocess_kernel": round(pre_marked, 5),
                               "bwd_main_kernel": round(main_marked, 5),
                               "ms_per_step": round(staged_ms, 5)},
-        "roofline": {"kernel": MAIN_KERNEL.get(name, "main kernel"), "bound": "mfma",
+        # the kernel behind the main stage (key "bwd_main_kernel" of the times)
+        "roofline": {"kernel": "bwd_reg_kernel" if F.plan_of(p).kernel == F.KERNEL_REG
+                     else "bwd_main_kernel", "bound": "mfma",
                      "achieved": round(main_tflops, 3),
                      "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(main_tflops / FP16_PEAK_TFLOPS, 5),
@@ -386,7 +381,7 @@ def measure(torch, lib, F, hip, name, steps, warmup, deterministic, dtype="fp16"
 
 
 def run_all(torch, lib, F, hip, args):
-    """Every BASELINE config: one JSON line each (GPU figures, the whole
+    """Every configuration P1-P5: one JSON line each (GPU figures, the whole
     config's CPU oracle backward), then a markdown table on stderr."""
     rows = []
     for name in ("P1", "P2", "P3", "P4", "P5"):
@@ -425,7 +420,7 @@ def main():
                          "0.3 s of GPU work, which brings the clocks to their steady state")
     ap.add_argument("--config", default="P3", choices=sorted(CONFIGS))
     ap.add_argument("--shape", default=None, metavar="B,Hq,Hkv,S,D,causal|full",
-                    help="time this shape instead of a BASELINE config (a diagnostic line, "
+                    help="time this shape instead of a configuration (a diagnostic line, "
                          "not the headline)")
     ap.add_argument("--dtype", default="fp16", choices=["fp16", "bf16"],
                     help="the inputs' 16-bit type (a diagnostic line; the headline is fp16)")
