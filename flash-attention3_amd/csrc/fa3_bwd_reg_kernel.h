@@ -27,11 +27,11 @@
 // S8192 D64 full 1 780 us against 1 606, B2 H16 S4096 D128 full 837 against
 // 750).  Against bwd_main_kernel a step also moves no P / dS through LDS
 // and a streamed tile serves 128 resident rows instead of 64, half the L2
-// traffic.  Measured against it (every launch on it before, one box), whole
-// backwards: B2 H16 S8192 D64 full 1 977 -> 1 631 us, B2 Hq32 Hkv8 S4096 D128
-// causal 947 -> 831, B1 Hq32 Hkv1 S4096 D128 causal 485 -> 437, B2 Hq32 Hkv8
-// S2048 D128 BSHD bf16 causal 255 -> 225, B4 H16 S1024 D128 causal bf16 90.5
-// -> 69.2, B2 H12 S1664 D64 full 77.1 -> 64.8.
+// traffic.  Measured against it (both in turn on one GPU), whole backwards:
+// B2 H16 S8192 D64 full 1 984 -> 1 624 us, B2 Hq32 Hkv8 S4096 D128 causal 963
+// -> 845, B1 Hq32 Hkv1 S4096 D128 causal 493 -> 442, B2 Hq32 Hkv8 S2048 D128
+// BSHD bf16 causal 257 -> 230, B4 H16 S1024 D128 causal bf16 92.6 -> 69.9, B2
+// H12 S1664 D64 full 77.8 -> 64.9.
 // Small launches are limited by one wave's chain (a wave alone on its SIMD
 // runs a 32 x 32 step in ~2 600 cycles, 1 024 of them MFMA), so launches
 // with few jobs stay with bwd_main_kernel (reg_plan, fa3_bwd_main.hip).

@@ -74,10 +74,10 @@ inline void set_job_map(FusedArgs& a, double longest = 0.0, double share = 1.0, 
 // n_groups set).  Always position by position across an XCD's groups, longest
 // jobs first: the hardware deals the jobs out in this order, and with small
 // workgroups a late long job costs more than the L2 gains from one group at a
-// time (B2 Hq32 Hkv8 S4096 D128 causal 1 029 -> 866 us, B4 H16 S1024 95.9 ->
-// 71.4, B4 H16 S2048 267.8 -> 240.7, B1 H16 S8192 783 -> 771; full attention,
-// B2 H12 S1664 D64 70.9 -> 63.8, B2 H16 S8192 D64 equal though five times the
-// algorithmic bytes are fetched).
+// time (bf16: B2 Hq32 Hkv8 S4096 D128 causal 914 -> 798 us, B4 H16 S1024 80.5
+// -> 70.1, B4 H16 S2048 261.5 -> 230.7, B1 H16 S8192 771 -> 755; full attention,
+// B2 H12 S1664 D64 68.3 -> 61.4, B2 H16 S8192 D64 1 521 -> 1 541, where five
+// times the algorithmic bytes are fetched).
 // Groups cut into parts of one job have no order inside an XCD: all roles and
 // lengths come mixed, group after group.  With three heads per dKV job or more,
 // which is then several times as long as a dQ job, the positions run across

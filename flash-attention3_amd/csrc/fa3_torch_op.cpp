@@ -2,9 +2,9 @@
 // workspace and launch of one backward in C++.
 //
 // What bounds the op at small sizes is the host, not the GPU: B2 H8 S256 D64
-// took 29.3 us a call, 7 of them in torch's dispatch and the rest in the
+// took 30.1 us a call, 7 of them in torch's dispatch and the rest in the
 // Python body (three checks, five allocations, a device guard, a ctypes call),
-// against ~9 us of GPU time.  With this body a call takes 20.4 us.  The op's
+// against ~9 us of GPU time.  With this body a call takes 21.1 us.  The op's
 // registration, autograd behaviour, fake implementation and argument checks
 // stay in Python; only the body below the checks moved.
 //

@@ -1,11 +1,11 @@
-"""Per-workgroup timeline of the main kernel (BASELINE configs P1-P5).
+"""Per-workgroup timeline of bwd_main_kernel (configurations P1-P5).
 
-Runs one BASELINE config with the timeline build of the library
+Runs one configuration with the timeline build of the library
 (``make -C flash-attention3_amd timeline`` -> lib/libshaobo_fa3_bwd_timeline.so,
-the main kernel compiled with -DFA3_TIMELINE) and prints a markdown summary of
+bwd_main_kernel compiled with -DFA3_TIMELINE) and prints a markdown summary of
 where each unit's time goes:
 
-    python flash-attention3_amd/timeline.py --config P3 [--raw gpurun_out/tl_P3.npy]
+    python flash-attention3_amd/timeline.py --config P3 [--raw tl_P3.npy]
 
 Stamps (s_memrealtime, 100 MHz) per workgroup: its entry; per unit u < 4: unit
 start, resident tiles landed, loop start, last step done, unit end (stores
@@ -15,7 +15,10 @@ of the persistent plan (P4, P5) runs many jobs: its first three go to units
 timed launch is the main kernel alone (the stage entry) after a full call
 filled the row statistics; the instrumented kernel waits for its stores at
 each unit end, so its unit gaps and epilogues run a little long.  The timeline
-build is a diagnostic: the product library compiles none of the stamps.
+build is a diagnostic: the product library compiles none of the stamps, and
+runs bwd_reg_kernel where the timeline build (which has no stamps in it) runs
+bwd_main_kernel's persistent plan -- P4 and P5 among them, whose timeline shows
+the kernel they ran before.
 """
 import argparse
 import ctypes

@@ -1,6 +1,6 @@
 // CPU oracle for the FA3 backward -- TEST INFRASTRUCTURE ONLY.
 //
-// This library is the checker the GPU path is compared against.  Only the
+// This library is the oracle the GPU path is compared against.  Only the
 // tests, __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it;
 // the shipped library (flash-attention3_amd/) never links or calls it.
 //
@@ -19,7 +19,7 @@
 //   dS      = P * (dP - delta_i) * scale                            :190
 //   dQ = dS K,  dK += dS^T Q,  dV += P^T dO  (GQA kv = h / (Hq/Hkv)) :166,196-198
 //   lse_i   = max_i * scale + ln(sum_i)                 full_bwd_correctness.cpp:229-233
-// Inputs (the build's own): Q, K, V, dO ~ N(0,1) from a
+// Inputs: Q, K, V, dO ~ N(0,1) from a
 // seeded splitmix64 + Box-Muller stream, rounded to fp16; and the reference's
 // deterministic pattern, generate_full_bwd_golden.py:135-151.  The *_fmt
 // entry points also take bf16 tensors (the build's bf16 extension; the

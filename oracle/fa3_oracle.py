@@ -3,7 +3,7 @@
 Loads oracle/lib/libfa3_oracle.so (a restatement of the reference's fp32 CPU
 golden, reference scripts/generate_full_bwd_golden.py:143-219; see
 fa3_bwd_oracle.cpp for the formula-by-formula citations).  Used by tests/,
-__graft_entry__.smoke() and bench.py's cpu_baseline leg as the checker; never
+__graft_entry__.smoke() and bench.py's cpu_baseline leg; never
 by the shipped library.
 
 Also holds the reference's five comparison metrics and gates
@@ -189,15 +189,15 @@ def metrics(actual, expected):
     }
 
 
-# max|err|/max|ref| <= 1e-2 for dQ/dK/dV, delta within 1e-4 relative.
+# The bar: max|err|/max|ref| <= 1e-2 for dQ/dK/dV, delta within 1e-4 relative.
 GRAD_MAX_REL = 1e-2
 DELTA_REL = 1e-4
 
 
 def gates(name, m):
-    """(north_star_ok, reference_gate_ok).
+    """(max_rel_ok, reference_gate_ok).
 
-    North star: max|err|/max|ref| <= 1e-2 for dQ/dK/dV; delta within 1e-4
+    Bar: max|err|/max|ref| <= 1e-2 for dQ/dK/dV; delta within 1e-4
     relative (rel_l2 and max|err|/max|ref|).  Reference gates
     (src/full_bwd_correctness.cpp:471-500): delta max_abs <= 5e-5 and
     rel_l2 <= 1e-4; dK/dV max_abs <= 3e-2 and rel_l2 <= 3e-2; dQ max_abs <=

@@ -93,7 +93,7 @@ BF16_GRAD_MAX_REL = 1.2e-2
 
 
 def check(res, g, names=("delta", "dq", "dk", "dv"), sel=None, reference_gates=False):
-    """Assert the north-star bar (and optionally the reference's own gates)."""
+    """Assert the max|err| / max|ref| bar (and optionally the reference's own gates)."""
     report = {}
     for n in names:
         a, e = res[n], g[n]

@@ -165,7 +165,7 @@ def test_our_writer_reproduces_reference_cache(tmp_path, dims):
 def test_oracle_against_reference_cache(dims):
     """The oracle on the reference's deterministic pattern: its inputs equal
     the cache's .f16 files bit for bit, and its outputs meet the reference's
-    own gates (src/full_bwd_correctness.cpp:471-500) and the north-star bar
+    own gates (src/full_bwd_correctness.cpp:471-500) and the oracle bar
     against the tool's fp32 results; O differs by at most one fp16 ulp and the
     row statistics agree to fp32 rounding (numpy sums in another order)."""
     import fa3_oracle as O

@@ -1,7 +1,7 @@
 """The reference harness flow from a golden cache (src/full_bwd_correctness.cpp:
 186-233, 366-392, 471-500): load the cache, form LSE = max * scale + ln(sum),
 run shaobo_fa3_bwd_v2 -- and the dot_do_o -> dkv -> dq chain -- and compare
-with the cache's fp32 gradients under the reference's gates and the north-star
+with the cache's fp32 gradients under the reference's gates and the oracle
 bar."""
 import ctypes
 import os
@@ -102,7 +102,7 @@ def test_v2_on_reference_tool_cache(hq, hkv):
     """v2 on the inputs of a cache written by the reference's own tool
     (fixtures under tests/golden/reference_caches, made by
     tests/golden/make_reference_caches.py), against that tool's fp32
-    gradients, under the reference's gates and the north-star bar."""
+    gradients, under the reference's gates and the oracle bar."""
     log(f"[case] reference tool cache v2 Hq{hq} Hkv{hkv} S128")
     dims = dict(batch=1, heads_q=hq, heads_kv=hkv, seqlen=128, head_dim=128)
     path = os.path.join(HERE, "golden", "reference_caches", GC.cache_key(causal=1, **dims))

@@ -1,7 +1,7 @@
 """GPU parity of shaobo_fa3_bwd_v2 (and the legacy / component entries)
-against the CPU oracle, through the C ABI, on the BASELINE configs.
+against the CPU oracle, through the C ABI, on the configurations P1 .. P5 and others.
 
-Bar (north star): max|err|/max|ref| <= 1e-2 for dQ/dK/dV, delta within 1e-4
+Bar: max|err|/max|ref| <= 1e-2 for dQ/dK/dV, delta within 1e-4
 relative; the reference's own gates (src/full_bwd_correctness.cpp:471-500)
 are asserted too on its deterministic pattern inputs, for which its absolute
 bounds were designed.  The full-size configs compare every (batch, kv-head)

@@ -3,7 +3,7 @@
 Each case draws one combination of the options the parity tests cover one at
 a time -- fp16 / bf16, BHSD / BSHD, GQA ratio 1, 2 or 4, causal or full, head
 dim 64 or 128, batch 1 or 2, S = 128 .. 1024, deterministic flag -- checks it
-against the CPU oracle to the north-star bar and checks that a second call
+against the CPU oracle to its bar and checks that a second call
 gives bitwise the same dQ, dK, dV.
 """
 import random
