@@ -305,7 +305,9 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 //     aligned: even group counts from S 7168 above 1.1, multiples of 4 from S
 //     3072 above 1.17 (58 shapes: this kernel -3 to +14 %, 4.5 % slower on
 //     average; odd counts -25 to +9 %);
-//   x > 1.3: bwd_main_kernel, 8 to 100 % faster the fewer the jobs.
+//   x > 1.3: bwd_main_kernel.  Whole jobs are 8 to 100 % slower there the fewer
+//     they are; with every dKV job halved (both roles with one head) 1.3 .. 1.6
+//     is 5 to 18 % faster on average, single shapes up to 14 % slower.
 // A dKV job longer than a workgroup slot's share sets the launch's end: such
 // tiles run as two jobs of 64 keys, at ~10 % more per unit.  Causal, only the
 // longest tiles (B2 Hq32 Hkv8 S2048 D128, of 16 tiles 0 / 4 / 8 / 12 / 16
