@@ -300,11 +300,6 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 //     longer the sequence the worse (S 256, 512: -4 to -13 %; S 1024 .. 2047:
 //     -1 to -5 % below 1.12, +2 to +6 % above; S >= 2048: +1 to +19 %; S 128:
 //     +5 % above 1.12): those run bwd_main_kernel;
-//     D 64 causal with more heads, near the upper end and with long sequences:
-//     bwd_main_kernel, whose prologues weigh less there, if its job map is
-//     aligned: even group counts from S 7168 above 1.1, multiples of 4 from S
-//     3072 above 1.17 (58 shapes: this kernel -3 to +14 %, 4.5 % slower on
-//     average; odd counts -25 to +9 %);
 //   x > 1.3: bwd_main_kernel.  Whole jobs are 8 to 100 % slower there the fewer
 //     they are; with every dKV job halved (both roles with one head) 1.3 .. 1.6
 //     is 5 to 18 % faster on average, single shapes up to 14 % slower.
@@ -362,12 +357,6 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
             r.split_kv = r.split_q = 2;
             return r;
         }
-    }
-    if (d64 && p.causal && heads > 1) {
-        const int groups = p.batch * p.heads_kv;
-        if ((p.seqlen >= 7168 && x > 1.1 && groups % 2 == 0) ||
-            (p.seqlen >= 3072 && x > 1.17 && groups % 4 == 0))
-            return r;
     }
     r.on = true;
     const double slot = share / (p.head_dim == 64 ? 3 : 2);

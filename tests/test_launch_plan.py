@@ -72,12 +72,6 @@ RULES = [
     (2, 16, 4, 2688, 128, False, "reg kv2 q1 c1"),       # four (0.87)
     (1, 48, 8, 2944, 128, False, "reg kv1 q1 c1"),       # six (0.80)
     (4, 264, 44, 128, 128, False, "reg kv1 q1 c1"),      # S < 1024 (0.83)
-    # D 64 causal, several heads, long sequences: bwd_main_kernel near the upper end
-    (2, 16, 1, 7296, 64, True, "main c2"),               # (1.26)
-    (4, 16, 1, 3584, 64, True, "main c2"),               # group count a multiple of 4 (1.26)
-    (3, 8, 2, 4992, 64, True, "reg h29/39 q1 c1"),       # 6 groups (1.22)
-    (3, 8, 1, 9984, 64, True, "reg h57/78 q1 c1"),       # odd (1.23)
-    (1, 18, 9, 3584, 64, True, "reg h20/28 q1 c1"),      # (1.12)
 ]
 
 
