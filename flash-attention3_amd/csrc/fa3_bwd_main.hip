@@ -300,9 +300,16 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 //     longer the sequence the worse (S 256, 512: -4 to -13 %; S 1024 .. 2047:
 //     -1 to -5 % below 1.12, +2 to +6 % above; S >= 2048: +1 to +19 %; S 128:
 //     +5 % above 1.12): those run bwd_main_kernel;
+//     D 64 causal with more heads and S >= 3072 is up to 9 % slower than
+//     bwd_main_kernel from 1.15 on (354 shapes, 4 % on average), but not than
+//     its unscaled instantiation (below), and stays;
 //   x > 1.3: bwd_main_kernel.  Whole jobs are 8 to 100 % slower there the fewer
 //     they are; with every dKV job halved (both roles with one head) 1.3 .. 1.6
 //     is 5 to 18 % faster on average, single shapes up to 14 % slower.
+// Launches below 1.3 with G > 1 that bwd_main_kernel runs take its unscaled
+// instantiation: S c in fp32 as in this kernel, not K c or Q c rounded (fp16
+// error against 64 bits 3.0e-4, scaled 3.7e-4), at the same speed (1 859 shapes
+// at D 128: 1.000 of the scaled one's time, up to 1.08).
 // A dKV job longer than a workgroup slot's share sets the launch's end: such
 // tiles run as two jobs of 64 keys, at ~10 % more per unit.  Causal, only the
 // longest tiles (B2 Hq32 Hkv8 S2048 D128, of 16 tiles 0 / 4 / 8 / 12 / 16
@@ -354,6 +361,7 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
         else most = p.seqlen >= 2048 ? 0.75 : p.seqlen >= 1024 || p.seqlen < 256 ? 1.12 : 1.3;
         if (x > most) {
             r.on = d64;
+            r.unscaled = group > 1;
             r.split_kv = r.split_q = 2;
             return r;
         }
@@ -374,7 +382,10 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
         if (d64 && heads > 1 && p.seqlen >= 512) most = 0.7;
         if (!d64 && heads == 2) {
             most = 1.14;
-            if (x > 0.9 && x <= most && p.seqlen >= 1024) r.on = false;
+            if (x > 0.9 && x <= most && p.seqlen >= 1024) {
+                r.on = false;
+                r.unscaled = true;
+            }
         }
         if (!d64 && heads > 3 && p.seqlen >= 1024) most = 0.8;
         if (x > most ||
@@ -442,6 +453,7 @@ void describe_launch(const BwdProblem& p, const WorkspacePlan& w, ShaoboFa3ExtPl
     o.kernel = reg.on ? SHAOBO_FA3_EXT_KERNEL_REG : SHAOBO_FA3_EXT_KERNEL_MAIN;
     o.split_plan = w.bal_m > 0 ? 1 : 0;
     o.chunks = chunks;
+    o.unscaled = reg.on || w.bal_m > 0 || !main_scaled(p.scale * kLog2e, reg.unscaled) ? 1 : 0;
     if (reg.on) {
         RegArgs r{};
         r.seqlen = p.seqlen;
@@ -586,9 +598,11 @@ hipError_t launch_backward(const BwdProblem& p, const BwdTensors& t, void* works
             launch_reg_race_check(r, reg, p.head_dim, p.causal, p.bf16, t.stream);
         else launch_reg_kernel<false>(r, reg, p.head_dim, p.causal, p.bf16, t.stream);
     }
-    else if (g_debug_kernels.load()) launch_race_check(a, p.head_dim, p.causal, p.bf16, t.stream);
-    else if (p.head_dim == 128) launch_dd<128, false>(a, p.causal, p.bf16, t.stream);
-    else launch_dd<64, false>(a, p.causal, p.bf16, t.stream);
+    else if (g_debug_kernels.load())
+        launch_race_check(a, p.head_dim, p.causal, p.bf16, reg.unscaled, t.stream);
+    else if (p.head_dim == 128)
+        launch_dd<128, false>(a, p.causal, p.bf16, reg.unscaled, t.stream);
+    else launch_dd<64, false>(a, p.causal, p.bf16, reg.unscaled, t.stream);
     err = hipGetLastError();
     if (err == hipSuccess && plan.hs_chunks > 0) {
         const dim3 rg((unsigned)((p.seqlen * (p.head_dim / 4) + 255) / 256),

@@ -6,10 +6,10 @@
 
 namespace fa3 {
 
-void launch_race_check(const FusedArgs& a, int head_dim, bool causal, bool bf16,
+void launch_race_check(const FusedArgs& a, int head_dim, bool causal, bool bf16, bool unscaled,
                        hipStream_t stream) {
-    if (head_dim == 128) launch_dd<128, true>(a, causal, bf16, stream);
-    else launch_dd<64, true>(a, causal, bf16, stream);
+    if (head_dim == 128) launch_dd<128, true>(a, causal, bf16, unscaled, stream);
+    else launch_dd<64, true>(a, causal, bf16, unscaled, stream);
 }
 
 void launch_reg_race_check(const RegArgs& a, RegPlan plan, int head_dim, bool causal, bool bf16,

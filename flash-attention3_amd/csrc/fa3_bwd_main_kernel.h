@@ -1939,10 +1939,15 @@ __global__ __launch_bounds__(256) void gqa_reduce_kernel(
     *(f16x4*)(dv + dst) = ov;
 }
 
+// Whether a default-plan launch multiplies its resident operands by the scale:
+// K c / Q c cannot overflow fp16 when c <= 1.
+inline bool main_scaled(float scale_log2, bool unscaled) { return scale_log2 <= 1.f && !unscaled; }
+
 // Instantiation of the main kernel for a launch: head dim, causal, 16-bit
 // type, split plan, scaled resident operands, race check.
+// unscaled: not the instantiations with scaled resident operands.
 template <int D, bool kDebug>
-void launch_dd(const FusedArgs& a, bool causal, bool bf16, hipStream_t stream) {
+void launch_dd(const FusedArgs& a, bool causal, bool bf16, bool unscaled, hipStream_t stream) {
     const dim3 grid(a.persist > 0 ? a.persist : a.n_groups * a.jobs_per_group);
     const dim3 block(kThreads);
     const bool split = a.bal_m > 0;  // causal only (plan_workspace)
@@ -1953,8 +1958,7 @@ void launch_dd(const FusedArgs& a, bool causal, bool bf16, hipStream_t stream) {
         const int sf = (int)(a.split_desc[i] >> 24);
         after = after || (sf != kNoShort && sf >= kShortAfter);
     }
-    // K c / Q c cannot overflow fp16 when c <= 1
-    const bool scaled = a.scale_log2 <= 1.f;
+    const bool scaled = main_scaled(a.scale_log2, unscaled);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, a); };
     // the default plan's job order: 2 head split (the plan set part_dk), 1
     // level by level (causal, G = 1), else 0
@@ -1993,7 +1997,7 @@ void launch_dd(const FusedArgs& a, bool causal, bool bf16, hipStream_t stream) {
 }  // namespace
 
 // The race-check instantiations (fa3_bwd_main_debug.hip).
-void launch_race_check(const FusedArgs& a, int head_dim, bool causal, bool bf16,
+void launch_race_check(const FusedArgs& a, int head_dim, bool causal, bool bf16, bool unscaled,
                        hipStream_t stream);
 
 }  // namespace fa3

@@ -49,7 +49,8 @@ namespace fa3 {
 // of a dQ job = 128 / split_q.  split_kv 0 (causal): the first `halved` of the
 // 128-key tiles, the longest, as two 64-key jobs, the others whole.
 struct RegPlan {
-    bool on = false;  // false: the launch runs bwd_main_kernel
+    bool on = false;  // false: the launch runs bwd_main_kernel,
+    bool unscaled = false;  // and its unscaled instantiation at every scale
     int split_kv = 1;
     int split_q = 1;
     int halved = 0;

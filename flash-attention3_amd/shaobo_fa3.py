@@ -109,8 +109,8 @@ KERNEL_MAIN, KERNEL_REG = range(2)
 class Plan(ctypes.Structure):
     """ShaoboFa3ExtPlan (include/shaobo_fa3_ext.h)."""
     _fields_ = [("struct_size", ctypes.c_uint32)] + [
-        (n, ctypes.c_int32) for n in ("kernel", "split_plan", "chunks", "jobs", "split_kv",
-                                      "halved", "split_q", "xcd_parts")]
+        (n, ctypes.c_int32) for n in ("kernel", "split_plan", "chunks", "jobs", "unscaled",
+                                      "split_kv", "halved", "split_q", "xcd_parts")]
 
 
 def _declare(lib):

@@ -137,6 +137,8 @@ typedef struct ShaoboFa3ExtPlan {
     int32_t split_plan;   /* 1: bwd_main_kernel's split plan (jobs in two pieces) */
     int32_t chunks;       /* dKV jobs per key tile and KV head; > 1: head split */
     int32_t jobs;         /* jobs of the launch (split plan: workgroups) */
+    int32_t unscaled;     /* 1: the softmax scale multiplies S in fp32; 0: the resident
+                           * K or Q, rounded to 16 bits again */
     /* bwd_reg_kernel only (0 otherwise) */
     int32_t split_kv;     /* dKV jobs of 128 / split_kv keys; 0: the first `halved` */
     int32_t halved;       /*   128-key tiles as two jobs of 64, the others whole */

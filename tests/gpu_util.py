@@ -24,7 +24,8 @@ def dev(t, torch, bshd=False):
 
 def launch_plan(B, Hq, Hkv, S, D, causal):
     """How the library runs a shape (shaobo_fa3_ext_bwd_v2_plan), as one word
-    group: "split" (bwd_main_kernel's split plan), "main c<chunks>", or of
+    group: "split" (bwd_main_kernel's split plan), "main c<chunks>" with
+    " unscaled" where its operands stay so at the default scale, or of
     bwd_reg_kernel "reg <dKV cut> q<split_q> c<chunks>", the dKV cut
     "kv<split_kv>" or, causal, "h<halved 128-key tiles>/<tiles>"."""
     p = F.plan_of(F.make_params(batch=B, seqlen=S, heads_q=Hq, heads_kv=Hkv, head_dim=D,
@@ -32,7 +33,7 @@ def launch_plan(B, Hq, Hkv, S, D, causal):
     if p.split_plan:
         return "split"
     if p.kernel == F.KERNEL_MAIN:
-        return f"main c{p.chunks}"
+        return f"main c{p.chunks}" + (" unscaled" if p.unscaled else "")
     cut = f"h{p.halved}/{S // 128}" if p.split_kv == 0 else f"kv{p.split_kv}"
     return f"reg {cut} q{p.split_q} c{p.chunks}"
 

@@ -370,7 +370,7 @@ def check_per_group(res, g):
 MANY_JOBS = [
     # Hq, Hkv, S, plan, at B1 D128 causal
     (16, 8, 4096, "reg h18/32 q1 c1"),   # bwd_reg_kernel, one dKV job per KV head
-    (8, 2, 4096, "main c4"),             # bwd_main_kernel, persistent (1024 jobs), head split
+    (8, 2, 4096, "main c4 unscaled"),    # bwd_main_kernel, persistent (1024 jobs), head split
     (4, 2, 8192, "main c1"),             # ... (768 jobs), one dKV job per KV head
 ]
 

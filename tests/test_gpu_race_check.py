@@ -52,8 +52,9 @@ RACE_CASES = [
     (3, 8, 8, 1024, 64, False, "fp16", "reg kv1 q1 c1"),
     (1, 2, 2, 512, 128, True, "bf16", "split"),             # bf16
     # bwd_main_kernel: head split and full attention
-    (2, 9, 3, 1536, 128, True, "fp16", "main c3"),          # 864 jobs: persistent head split
-    (1, 20, 5, 768, 128, False, "bf16", "main c4"),         # 480 jobs: head split, full
+    (2, 9, 3, 1536, 128, True, "fp16", "main c3 unscaled"),  # 864 jobs: persistent head split
+    (1, 12, 4, 1536, 128, True, "fp16", "main c3"),         # ... (576 jobs) with scaled operands
+    (1, 20, 5, 768, 128, False, "bf16", "main c4 unscaled"), # 480 jobs: head split, full
     (2, 6, 2, 1024, 64, False, "fp16", "main c3"),          # ... D 64
     (2, 8, 8, 1024, 128, False, "fp16", "main c1"),         # 512 jobs: one per workgroup, full
     (3, 5, 5, 1536, 128, False, "fp16", "main c1"),         # 720 jobs: persistent, full

@@ -32,15 +32,15 @@ def test_plan_arguments():
 RULES = [
     # B, Hq, Hkv, S, D, causal, plan; longest dKV job / a CU's share
     # one head per chunk: a dQ job is as long as a dKV job, as with G = 1
-    (1, 4, 1, 3968, 128, False, "main c4"),              # D 128 (1.18)
-    (1, 20, 5, 768, 128, False, "main c4"),              # (1.22)
+    (1, 4, 1, 3968, 128, False, "main c4 unscaled"),     # D 128 (1.18)
+    (1, 20, 5, 768, 128, False, "main c4 unscaled"),     # (1.22)
     (1, 44, 11, 384, 128, False, "reg kv2 q1 c4"),       # (1.11)
-    (1, 8, 2, 3584, 128, True, "main c4"),               # causal, S >= 2048 (1.26)
-    (2, 3, 1, 7808, 128, True, "main c3"),               # (0.79)
-    (2, 9, 3, 1536, 128, True, "main c3"),               # S >= 1024 (1.25)
+    (1, 8, 2, 3584, 128, True, "main c4 unscaled"),      # causal, S >= 2048 (1.26)
+    (2, 3, 1, 7808, 128, True, "main c3 unscaled"),      # (0.79)
+    (2, 9, 3, 1536, 128, True, "main c3 unscaled"),      # S >= 1024 (1.25)
     (3, 8, 1, 1280, 128, True, "reg h6/10 q1 c8"),       # (1.11)
     (1, 18, 3, 1920, 128, True, "reg h8/15 q1 c6"),      # (1.05)
-    (2, 60, 10, 128, 128, True, "main c6"),              # S < 256 (1.22)
+    (2, 60, 10, 128, 128, True, "main c6 unscaled"),     # S < 256 (1.22)
     (1, 36, 12, 768, 128, True, "reg h4/6 q1 c3"),       # between (1.16)
     (1, 20, 5, 768, 64, False, "reg kv2 q2 c4"),         # D 64 (1.22)
     (3, 24, 3, 256, 64, False, "reg kv2 q1 c8"),         # S < 512 (1.02)
@@ -63,8 +63,8 @@ RULES = [
     (13, 16, 8, 256, 64, False, "reg kv1 q1 c1"),        # S < 512 (0.70)
     # D 128 full: halved with two heads per dKV job from 1.14 on, with four from 0.8
     (8, 6, 3, 768, 128, False, "reg kv1 q1 c1"),         # two (1.02)
-    (2, 16, 1, 1152, 128, False, "main c8"),             # S >= 1024 (1.02)
-    (1, 34, 17, 1024, 128, False, "main c1"),            # (1.08)
+    (2, 16, 1, 1152, 128, False, "main c8 unscaled"),    # S >= 1024 (1.02)
+    (1, 34, 17, 1024, 128, False, "main c1 unscaled"),   # (1.08)
     (5, 4, 2, 2304, 128, False, "reg kv1 q1 c1"),        # 1.05 rounds (0.81)
     (7, 14, 7, 512, 128, False, "reg kv2 q1 c1"),        # S < 1024 (0.75)
     (1, 32, 16, 1024, 128, False, "reg kv2 q1 c1"),      # (1.14)
