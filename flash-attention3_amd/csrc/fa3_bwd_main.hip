@@ -329,6 +329,9 @@ WorkspacePlan plan_workspace(const BwdProblem& p) {
 //   D 64, more than one head, S >= 512: from 0.7 on (71 shapes of 0.7 .. 0.9,
 //     whole -> halved: S >= 1024 1.00, up to 1.13 -> 0.84, up to 0.90; S 512 ..
 //     1023 0.87 -> 0.74; shorter 0.75 -> 0.69, but some 18 % slower halved);
+//     two heads from 0.76 on, where halved dKV and dQ jobs fit one round of
+//     three workgroups per CU (0.76 .. 0.8: halved 0.85 of whole, 0.7 .. 0.76
+//     1.04);
 //   D 128, two heads: from 1.14 on, where the halved jobs are at most one per
 //     CU (above it whole 1.07, halved 0.82); of 0.9 .. 1.14 whole below S 1024
 //     (28 shapes, halved -> whole: 0.97, up to 1.11 -> 0.89, up to 1.02), and
@@ -379,7 +382,7 @@ RegPlan reg_plan(const BwdProblem& p, const WorkspacePlan& w) {
         const double rounds = (double)p.batch * p.heads_kv * (chunks + group) * (qt / 2) /
                               (2 * kHeadSplitCus);
         double most = 0.9;
-        if (d64 && heads > 1 && p.seqlen >= 512) most = 0.7;
+        if (d64 && heads > 1 && p.seqlen >= 512) most = heads == 2 ? 0.76 : 0.7;
         if (!d64 && heads == 2) {
             most = 1.14;
             if (x > 0.9 && x <= most && p.seqlen >= 1024) {

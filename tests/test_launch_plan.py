@@ -72,6 +72,9 @@ RULES = [
     (2, 16, 4, 2688, 128, False, "reg kv2 q1 c1"),       # four (0.87)
     (1, 48, 8, 2944, 128, False, "reg kv1 q1 c1"),       # six (0.80)
     (4, 264, 44, 128, 128, False, "reg kv1 q1 c1"),      # S < 1024 (0.83)
+    # D 64 full, two heads: from 0.76 on
+    (4, 4, 2, 3328, 64, False, "reg kv1 q1 c1"),         # (0.70)
+    (1, 32, 16, 1536, 64, False, "reg kv2 q1 c1"),       # (0.76)
 ]
 
 
